@@ -78,6 +78,7 @@ SIGNATURES = {
     'fk_convar_jvp': (ctypes.c_int, [_P, _P, _I32, _I32, _I32, _I32, _I32, _P, _I64, _P, _P, _P, _P]),
     'fk_wn_grad_rows': (ctypes.c_int, [_P, _I64, _I64, _P, _P, _P, _I32, _I32, _I32, _I64, _P]),
     'fk_wn_tangent': (ctypes.c_int, [_P, _P, _P, _I32, _I32, _I32, _P, _P, _I64, _P]),
+    'fk_wn_effective': (ctypes.c_int, [_P, _P, _P, _I32, _I32, _I32, _P, _I64, _P]),
     'fk_o_mean': (ctypes.c_int, [_P, _P, _I64, _I64, _P, _P, _P]),
     'fk_o_times_v': (ctypes.c_int, [_P, _P, _P, _P, _P, _I64, _I64, _P, _P, _P]),
     'fk_oh_times_u': (ctypes.c_int, [_P, _P, _P, _P, _P, _I64, _I64, ctypes.c_double, ctypes.c_double, _P, _P,

@@ -4,8 +4,8 @@
 // (tf.nn.l2_normalize) and s = exp(g) (exponential_norm) or g.  The gradient
 // kernels of this library differentiate with respect to k; these kernels map
 // such derivatives onto the trainable (v, g), and parameter directions
-// (v', g') onto directions in k.  Small elementwise work: one thread per
-// (row, layer, output channel).
+// (v', g') onto directions in k; fk_wn_effective forms the kernels k
+// themselves.
 #include "fk_common.h"
 
 namespace fk {
@@ -20,44 +20,130 @@ __device__ __forceinline__ WnLayer wn_layer(const int64_t* t, int l) {
   return WnLayer{t[4 * l], t[4 * l + 1], t[4 * l + 2], t[4 * l + 3]};
 }
 
-// Norm and scale of channel c of layer L.
-__device__ __forceinline__ void wn_norm(const float* v, const WnLayer& L, int64_t c, const float* g, int exp_norm,
-                                        float& n, float& s, bool& clamped) {
-  float ss = 0.0f;
-  for (int64_t i = 0; i < L.nin; ++i) {
-    const float x = v[L.koff + i * L.cout + c];
-    ss += x * x;
+// Threads of a workgroup over one (layer, tile of CT channels): channel
+// c = tile * CT + tid % CT, and the channel's nin values dealt to the G =
+// threads / CT groups tid / CT.  Neighbouring threads then read neighbouring
+// channels, so a wave's loads are contiguous (kernels are (..., cin, cout)).
+// What bounds these kernels is the chain of loads of one channel: with a
+// thread per channel it was nin (up to 576) dependent iterations, 213 us for
+// one row of the 4x4 depth-5 32-channel network and 519 us for 256 rows of
+// the 12x12 depth-10 one (1.6 TB/s); dealt to the groups, WN_FIGS.
+constexpr int WN_THREADS = 256;
+
+struct WnTile {
+  int CT, G, grp;
+  int64_t c;
+  bool live;
+};
+
+__device__ __forceinline__ int wn_tile_channels(const WnLayer& L) { return L.cout < 64 ? (int)L.cout : 64; }
+
+__device__ __forceinline__ WnTile wn_tile(const WnLayer& L, int64_t tile) {
+  WnTile t;
+  t.CT = wn_tile_channels(L);
+  t.G = WN_THREADS / t.CT;
+  t.grp = (int)threadIdx.x / t.CT;
+  t.c = tile * t.CT + (int)threadIdx.x % t.CT;
+  t.live = t.grp < t.G && t.c < L.cout;
+  return t;
+}
+
+// Sum over the groups of a channel, in group order (FP64, deterministic);
+// every thread of the channel gets it.  red: WN_THREADS doubles.
+__device__ __forceinline__ double wn_group_sum(double x, const WnTile& t, double* red) {
+  __syncthreads();
+  red[threadIdx.x] = x;
+  __syncthreads();
+  const int col = (int)threadIdx.x % t.CT;
+  double s = 0.0;
+  for (int k = 0; k < t.G; ++k) s += red[k * t.CT + col];
+  return s;
+}
+
+// Norm and scale of the thread's channel.
+__device__ __forceinline__ void wn_norm(const float* __restrict__ v, const WnLayer& L, const WnTile& t,
+                                        const float* __restrict__ g, int exp_norm, double* red, float& n, float& s,
+                                        bool& clamped) {
+  double ss = 0.0;
+  if (t.live) {
+    const float* p = v + L.koff + t.c;
+#pragma unroll 4
+    for (int64_t i = t.grp; i < L.nin; i += t.G) {
+      const double x = p[i * L.cout];
+      ss += x * x;
+    }
   }
-  clamped = ss < 1e-12f;
-  n = sqrtf(clamped ? 1e-12f : ss);
-  s = exp_norm ? expf(g[L.goff + c]) : g[L.goff + c];
+  ss = wn_group_sum(ss, t, red);
+  clamped = (float)ss < 1e-12f;
+  n = clamped ? sqrtf(1e-12f) : (float)sqrt(ss);
+  s = 0.0f;
+  if (t.live) s = exp_norm ? expf(g[L.goff + t.c]) : g[L.goff + t.c];
+}
+
+// v . x over the thread's channel (x: a row of d/dk or a direction).
+__device__ __forceinline__ float wn_dot(const float* __restrict__ v, const float* __restrict__ x, const WnLayer& L,
+                                        const WnTile& t, double* red) {
+  double dot = 0.0;
+  if (t.live) {
+    const int64_t q0 = L.koff + t.c;
+#pragma unroll 4
+    for (int64_t i = t.grp; i < L.nin; i += t.G) dot += (double)v[q0 + i * L.cout] * x[q0 + i * L.cout];
+  }
+  return (float)wn_group_sum(dot, t, red);
+}
+
+// The kernels of wrapped layers, k = v / n * s, one workgroup per (tile of
+// channels, layer); every other entry is copied beforehand.
+__global__ __launch_bounds__(WN_THREADS) void wn_effective_kernel(const float* __restrict__ v,
+                                                                  const float* __restrict__ g,
+                                                                  const int64_t* __restrict__ layers, int exp_norm,
+                                                                  float* __restrict__ out) {
+  __shared__ double red[WN_THREADS];
+  const WnLayer L = wn_layer(layers, blockIdx.y);
+  if ((int64_t)blockIdx.x * wn_tile_channels(L) >= L.cout) return;
+  const WnTile t = wn_tile(L, blockIdx.x);
+  float n, s;
+  bool clamped;
+  wn_norm(v, L, t, g, exp_norm, red, n, s, clamped);
+  if (!t.live) return;
+#pragma unroll 4
+  for (int64_t i = t.grp; i < L.nin; i += t.G) {
+    const int64_t q = L.koff + i * L.cout + t.c;
+    out[q] = v[q] / n * s;
+  }
 }
 
 // In place on rows (nrows, ld): row[:P] holds d/dk on entry; on exit the
 // kernel entries of every wrapped layer hold d/dv and row[P + goff + c] holds
 // d/dg.  dv_i = s/n (dk_i - v_i (v.dk)/n^2) (s/n dk_i when the norm is
-// clamped), dg = s/n (v.dk) for exponential_norm, (v.dk)/n otherwise.
-__global__ void wn_grad_rows_kernel(float* __restrict__ rows, int64_t nrows, int64_t ld,
-                                    const float* __restrict__ v, const float* __restrict__ g,
-                                    const int64_t* __restrict__ layers, int exp_norm, int64_t P) {
+// clamped), dg = s/n (v.dk) for exponential_norm, (v.dk)/n otherwise.  A
+// workgroup takes rows blockIdx.z, blockIdx.z + gridDim.z, ... of one (tile,
+// layer), so the norm is computed once for them.
+__global__ __launch_bounds__(WN_THREADS) void wn_grad_rows_kernel(float* __restrict__ rows, int64_t nrows, int64_t ld,
+                                                                  const float* __restrict__ v,
+                                                                  const float* __restrict__ g,
+                                                                  const int64_t* __restrict__ layers, int exp_norm,
+                                                                  int64_t P) {
+  __shared__ double red[WN_THREADS];
   const WnLayer L = wn_layer(layers, blockIdx.y);
-  const int64_t per_block = (int64_t)blockDim.x;
-  const int64_t idx = (int64_t)blockIdx.x * per_block + threadIdx.x;
-  const int64_t r = idx / L.cout, c = idx - (idx / L.cout) * L.cout;
-  if (r >= nrows) return;
+  if ((int64_t)blockIdx.x * wn_tile_channels(L) >= L.cout) return;
+  const WnTile t = wn_tile(L, blockIdx.x);
   float n, s;
   bool clamped;
-  wn_norm(v, L, c, g, exp_norm, n, s, clamped);
-  float* row = rows + r * ld;
-  float dot = 0.0f;
-  for (int64_t i = 0; i < L.nin; ++i) dot += v[L.koff + i * L.cout + c] * row[L.koff + i * L.cout + c];
+  wn_norm(v, L, t, g, exp_norm, red, n, s, clamped);
   const float sn = s / n;
-  const float proj = clamped ? 0.0f : dot / (n * n);
-  for (int64_t i = 0; i < L.nin; ++i) {
-    const int64_t q = L.koff + i * L.cout + c;
-    row[q] = sn * (row[q] - v[q] * proj);
+  for (int64_t r = blockIdx.z; r < nrows; r += gridDim.z) {
+    float* row = rows + r * ld;
+    const float dot = wn_dot(v, row, L, t, red);
+    if (!t.live) continue;
+    const float proj = clamped ? 0.0f : dot / (n * n);
+#pragma unroll 4
+    for (int64_t i = t.grp; i < L.nin; i += t.G) {
+      const int64_t q = L.koff + i * L.cout + t.c;
+      row[q] = sn * (row[q] - v[q] * proj);
+    }
+    if (t.grp == 0) row[P + L.goff + t.c] = exp_norm ? sn * dot : dot / n;
   }
-  row[P + L.goff + c] = exp_norm ? sn * dot : dot / n;
 }
 
 // t_eff (P) from a direction t over (v, g): kernel entries
@@ -68,24 +154,28 @@ __global__ void wn_copy_kernel(const float* __restrict__ t, float* __restrict__ 
   if (q < P) out[q] = t[q];
 }
 
-__global__ void wn_tangent_kernel(const float* __restrict__ v, const float* __restrict__ g,
-                                  const int64_t* __restrict__ layers, int exp_norm, const float* __restrict__ t,
-                                  float* __restrict__ out, int64_t P) {
+__global__ __launch_bounds__(WN_THREADS) void wn_tangent_kernel(const float* __restrict__ v,
+                                                                const float* __restrict__ g,
+                                                                const int64_t* __restrict__ layers, int exp_norm,
+                                                                const float* __restrict__ x, float* __restrict__ out,
+                                                                int64_t P) {
+  __shared__ double red[WN_THREADS];
   const WnLayer L = wn_layer(layers, blockIdx.y);
-  const int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= L.cout) return;
+  if ((int64_t)blockIdx.x * wn_tile_channels(L) >= L.cout) return;
+  const WnTile t = wn_tile(L, blockIdx.x);
   float n, s;
   bool clamped;
-  wn_norm(v, L, c, g, exp_norm, n, s, clamped);
-  float dot = 0.0f;
-  for (int64_t i = 0; i < L.nin; ++i) dot += v[L.koff + i * L.cout + c] * t[L.koff + i * L.cout + c];
+  wn_norm(v, L, t, g, exp_norm, red, n, s, clamped);
+  const float dot = wn_dot(v, x, L, t, red);
+  if (!t.live) return;
   const float sn = s / n;
   const float proj = clamped ? 0.0f : dot / (n * n);
-  const float tg = t[P + L.goff + c];
-  for (int64_t i = 0; i < L.nin; ++i) {
-    const int64_t q = L.koff + i * L.cout + c;
+  const float tg = x[P + L.goff + t.c];
+#pragma unroll 4
+  for (int64_t i = t.grp; i < L.nin; i += t.G) {
+    const int64_t q = L.koff + i * L.cout + t.c;
     const float dkdg = exp_norm ? v[q] * sn : v[q] / n;
-    out[q] = sn * (t[q] - v[q] * proj) + dkdg * tg;
+    out[q] = sn * (x[q] - v[q] * proj) + dkdg * tg;
   }
 }
 
@@ -103,9 +193,12 @@ int fk_wn_grad_rows(float* rows, int64_t nrows, int64_t ld, const float* params,
   FK_REQUIRE(rows && params && g && layers, "fk_wn_grad_rows: null pointer");
   FK_REQUIRE(ld >= n_params, "fk_wn_grad_rows: row stride shorter than the parameters");
   FK_REQUIRE(n_layers <= 65535, "fk_wn_grad_rows: too many layers");
-  const int64_t threads = nrows * (int64_t)max_cout;
-  hipLaunchKernelGGL(wn_grad_rows_kernel, dim3((unsigned)div_up(threads, 256), (unsigned)n_layers), dim3(256), 0,
-                     (hipStream_t)stream, rows, nrows, ld, params, g, layers, exp_norm, n_params);
+  // few rows: a workgroup per row; many: the rows dealt to as many workgroups
+  // as keep 16 of them per CU, so that the norms are not recomputed per row
+  const int64_t most = 1 + 16LL * device_cu_count() / n_layers;
+  hipLaunchKernelGGL(wn_grad_rows_kernel,
+                     dim3((unsigned)div_up(max_cout, 64), (unsigned)n_layers, (unsigned)(nrows < most ? nrows : most)),
+                     dim3(WN_THREADS), 0, (hipStream_t)stream, rows, nrows, ld, params, g, layers, exp_norm, n_params);
   FK_CHECK_LAUNCH();
   return FK_OK;
 }
@@ -121,8 +214,25 @@ int fk_wn_tangent(const float* params, const float* g, const int64_t* layers, in
     FK_CHECK_LAUNCH();
   }
   if (n_layers == 0) return FK_OK;
-  hipLaunchKernelGGL(wn_tangent_kernel, dim3((unsigned)div_up(max_cout, 64), (unsigned)n_layers), dim3(64), 0, s,
-                     params, g, layers, exp_norm, t, t_eff, n_params);
+  hipLaunchKernelGGL(wn_tangent_kernel, dim3((unsigned)div_up(max_cout, 64), (unsigned)n_layers), dim3(WN_THREADS), 0,
+                     s, params, g, layers, exp_norm, t, t_eff, n_params);
+  FK_CHECK_LAUNCH();
+  return FK_OK;
+}
+
+int fk_wn_effective(const float* params, const float* g, const int64_t* layers, int32_t n_layers, int32_t max_cout,
+                    int32_t exp_norm, float* effective, int64_t n_params, void* stream) {
+  FK_REQUIRE(n_layers >= 0 && max_cout >= 1 && n_params >= 0, "fk_wn_effective: bad sizes");
+  FK_REQUIRE(params && effective && (n_layers == 0 || (g && layers)), "fk_wn_effective: null pointer");
+  FK_REQUIRE(n_layers <= 65535, "fk_wn_effective: too many layers");
+  hipStream_t s = (hipStream_t)stream;
+  if (n_params > 0) {
+    hipLaunchKernelGGL(wn_copy_kernel, dim3(div_up(n_params, 256)), dim3(256), 0, s, params, effective, n_params);
+    FK_CHECK_LAUNCH();
+  }
+  if (n_layers == 0) return FK_OK;
+  hipLaunchKernelGGL(wn_effective_kernel, dim3((unsigned)div_up(max_cout, 64), (unsigned)n_layers), dim3(WN_THREADS),
+                     0, s, params, g, layers, exp_norm, effective);
   FK_CHECK_LAUNCH();
   return FK_OK;
 }

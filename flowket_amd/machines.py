@@ -195,6 +195,12 @@ class ConvNetAutoregressive2D:
         * exp(g) per output channel (wrappers.py:123-135)."""
         if not self.weights_normalization:
             return self.params
+        if self.device.type == 'cuda':
+            tab, nl, mc = self._wn_table()
+            eff = torch.empty(self.n_params, dtype=torch.float32, device=self.device)
+            _lib.call('fk_wn_effective', _lib.ptr(self.params), _lib.ptr(self.wn_g), _lib.ptr(tab), nl, mc,
+                      int(self.exponential_norm), _lib.ptr(eff), self.n_params, _lib.stream_ptr())
+            return eff
         parts, gi = [], 0
         p = self.params
         for idx, off, kshape in self._wn_layer_views(p):
@@ -436,16 +442,20 @@ class ConvNetAutoregressive2D:
         respect to the effective kernels and biases (P floats): scale *
         Re[O^H u] for u = cot[:,0] + i cot[:,1], through fk_convar_vjp (one
         batched backward pass, O never formed)."""
+        grad = torch.empty(self.n_params, dtype=torch.float32, device=self.device)
+        self._vjp_into(grad, x, cot, scale, stream)
+        return grad
+
+    def _vjp_into(self, grad, x, cot, scale, stream):
+        """vjp_effective into the first n_params floats of ``grad``."""
         _lib.require_gpu()
         spins = self._spins(x)
         B = spins.shape[0]
         cot = torch.as_tensor(cot).to(self.device, torch.float32).reshape(B, 2).contiguous()
-        grad = torch.empty(self.n_params, dtype=torch.float32, device=self.device)
         ws = self._implicit_workspace('vjp', B)
         _lib.call('fk_convar_vjp', _lib.ptr(self.effective_params().contiguous()), self.H, self.W, self.depth,
                   self.num_of_channels, _ACT[self.activation], _lib.ptr(spins), B, _lib.ptr(cot), float(scale),
                   _lib.ptr(ws), _lib.ptr(grad), None, _lib.stream_ptr(stream))
-        return grad
 
     def jvp_effective(self, x, tangent, stream=None):
         """(B, 2) float32: (dRe log psi_b . t, dIm log psi_b . t) for a
@@ -517,11 +527,11 @@ class ConvNetAutoregressive2D:
         """scale * Re[O^H u] (u = cot[:,0] + i cot[:,1]) over the trainable
         values (n_trainable floats), O never formed: fk_convar_vjp, then the
         weight-normalisation chain rule."""
-        g = self.vjp_effective(x, cot, scale, stream)
         if not self.weights_normalization:
-            return g
-        out = torch.zeros(self.n_trainable, dtype=torch.float32, device=self.device)
-        out[:self.n_params] = g
+            return self.vjp_effective(x, cot, scale, stream)
+        # the chain rule writes every g entry, so nothing needs clearing
+        out = torch.empty(self.n_trainable, dtype=torch.float32, device=self.device)
+        self._vjp_into(out, x, cot, scale, stream)
         self._wn_rows(out, 1)
         return out
 

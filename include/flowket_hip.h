@@ -371,7 +371,9 @@ int fk_convar_jvp(const float* params, const float* tangent, int32_t H,
  *                    d/dk in [0, P) becomes d/dv in the kernel slots, and
  *                    d/dg is written at P + goff + c (the trainable order
  *                    [params | g]).
- *   fk_wn_tangent:   t_eff (P) = dk for a direction t over [params | g]. */
+ *   fk_wn_tangent:   t_eff (P) = dk for a direction t over [params | g].
+ *   fk_wn_effective: effective (P) = params with every wrapped layer's kernel
+ *                    slots holding k instead of v. */
 int fk_wn_grad_rows(float* rows, int64_t nrows, int64_t ld,
                     const float* params, const float* g, const int64_t* layers,
                     int32_t n_layers, int32_t max_cout, int32_t exp_norm,
@@ -380,6 +382,9 @@ int fk_wn_tangent(const float* params, const float* g, const int64_t* layers,
                   int32_t n_layers, int32_t max_cout, int32_t exp_norm,
                   const float* t, float* t_eff, int64_t n_params,
                   void* stream);
+int fk_wn_effective(const float* params, const float* g, const int64_t* layers,
+                    int32_t n_layers, int32_t max_cout, int32_t exp_norm,
+                    float* effective, int64_t n_params, void* stream);
 
 /* ---------------------------------------------------------------------------
  * Stochastic reconfiguration on the implicit S = Re[(O-Obar)^H (O-Obar)]/B

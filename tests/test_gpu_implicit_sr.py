@@ -275,3 +275,32 @@ def test_sr_training_lowers_the_exact_energy(jvp):
     e1 = ev.energy_observable.current_energy.real
     assert e1 < e0 - 5.0, (e0, e1)
     assert e1 > -44.9139328337 - 1e-6   # variational bound
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('exp_norm', [True, False])
+@pytest.mark.parametrize('depth,channels', [(2, 2), (3, 10), (4, 20), (3, 64)])
+def test_wn_effective_kernels(depth, channels, exp_norm):
+    """fk_wn_effective against the FP64 transform over channel counts that
+    divide the workgroup unevenly, with one all-zero channel (the clamped
+    norm).  Tolerance: the FP64 norm is rounded once and v / n * s rounds
+    twice, exp is good to 2 ulp: 4 ulp = 2.4e-7 relative."""
+    import flowket_amd as fk
+    m = fk.ConvNetAutoregressive2D((3, 3), depth=depth, num_of_channels=channels, weights_normalization=True,
+                                   exponential_norm=exp_norm, seed=7)
+    flat = m.params.cpu().clone()
+    kshape = m.shapes[0][0]
+    flat[:int(np.prod(kshape))].reshape(kshape)[..., 0] = 0.0
+    m.set_params(flat)
+    got = m.effective_params().cpu().double().numpy()
+    g, off, goff = m.wn_g.cpu().double().numpy(), 0, 0
+    p = flat.double().numpy()
+    for k, (ks, bs) in enumerate(m.shapes):
+        nk = int(np.prod(ks))
+        ref = p[off:off + nk]
+        if k < len(m.shapes) - 1:
+            ref = ocn.weight_norm(ref.reshape(ks), g[goff:goff + bs[0]], exp_norm).reshape(-1)
+            goff += bs[0]
+        np.testing.assert_allclose(got[off:off + nk], ref, rtol=2.4e-7, atol=0)
+        np.testing.assert_array_equal(got[off + nk:off + nk + bs[0]], p[off + nk:off + nk + bs[0]])
+        off += nk + bs[0]
