@@ -46,62 +46,156 @@ __device__ __forceinline__ float wave_sum(float v) {
   return v;
 }
 
+// lncosh(x + iy) with one exponential: of e^{x-|x|} and e^{-x-|x|} one is 1
+// and the other e^{-2|x|}, the e2 of lncosh_re.
+__device__ __forceinline__ void lncosh(float x, float y, float& re, float& im) {
+  const float ax = fabsf(x);
+  const float e = expf(-2.0f * ax);
+  re = ax - 0.69314718055994531f + 0.5f * log1pf(e * e + 2.0f * e * cosf(2.0f * y));
+  const float e1 = x >= 0.0f ? 1.0f : e, e2 = x >= 0.0f ? e : 1.0f;
+  float sy, cy;
+  sincosf(y, &sy, &cy);
+  im = atan2f((e1 - e2) * sy, (e1 + e2) * cy);
+}
+
 // log psi of configurations: rows of `spins` or (sample, connection) pairs
 // applied with the connection table (kind as fk_find_conn).
-__global__ __launch_bounds__(256) void rbm_log_psi_kernel(RbmParams p, const int8_t* __restrict__ spins,
-                                                          const int32_t* __restrict__ pairs,
-                                                          const int64_t* __restrict__ m_dev, int64_t m_count,
-                                                          int conn_kind, const int32_t* __restrict__ conn_a,
-                                                          const int32_t* __restrict__ conn_b,
-                                                          float* __restrict__ out) {
-  const int lane = threadIdx.x & 63;
-  const int64_t m = (int64_t)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
+//
+// A wave evaluates K consecutive configurations, hidden units over its lanes
+// (HPL per lane at a time): a weight read once serves K of them.  With K = 1
+// the 131 KB of weights of the 8x8 alpha-4 RBM came from L2 for every
+// configuration (266k of them in 2671 us, 13 TB/s); eight per wave take
+// 830 us, most of it the lncosh of 256 hidden units each.
+// The spins of the K configurations sit in LDS as floats, in chunks of
+// RBM_NJ sites, so four sites of one configuration are one broadcast read.
+// theta is summed over the sites in order and log psi over a lane's hidden
+// units in order, whatever K and HPL: results do not depend on them.
+constexpr int RBM_NJ = 64, RBM_WAVES = 4;
+
+template <int K, int HPL>
+__global__ __launch_bounds__(64 * RBM_WAVES, 4) void rbm_log_psi_kernel(
+    RbmParams p, const int8_t* __restrict__ spins, const int32_t* __restrict__ pairs,
+    const int64_t* __restrict__ m_dev, int64_t m_count, int conn_kind, const int32_t* __restrict__ conn_a,
+    const int32_t* __restrict__ conn_b, float* __restrict__ out) {
+  __shared__ f32x4 s_spin[RBM_WAVES][K][RBM_NJ / 4];
+  // (the wave index made uniform: its configurations' addresses stay scalar)
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int64_t m0 = ((int64_t)blockIdx.x * RBM_WAVES + wave) * K;
   int64_t M = m_dev ? *m_dev : m_count;
   if (M > m_count) M = m_count;
-  if (m >= M) return;
-  int64_t b = m;
-  int c = 0;
-  if (pairs) {
-    b = pairs[2 * m];
-    c = pairs[2 * m + 1];
+  if (m0 >= M) return;  // waves are independent: no barrier below
+  const int8_t* row[K];
+  int fa[K], fb[K];
+#pragma unroll
+  for (int k = 0; k < K; ++k) {
+    const int64_t m = m0 + k < M ? m0 + k : M - 1;  // the last wave repeats the last configuration
+    int64_t b = m;
+    int c = 0;
+    if (pairs) {
+      b = pairs[2 * m];
+      c = pairs[2 * m + 1];
+    }
+    row[k] = spins + b * p.N;
+    fa[k] = fb[k] = -1;
+    if (c > 0) {
+      fa[k] = conn_a[c];
+      fb[k] = (conn_kind == FK_CONN_FLIP) ? -1 : conn_b[c];
+    }
   }
-  const int8_t* row = spins + b * p.N;
-  int fa = -1, fb = -1;
-  if (c > 0) {
-    fa = conn_a[c];
-    fb = (conn_kind == FK_CONN_FLIP) ? -1 : conn_b[c];
-  }
-  auto spin = [&](int j) -> float {
-    int8_t v = row[j];
+  auto spin = [&](int k, int j) -> float {
+    int8_t v = row[k][j];
     if (conn_kind == FK_CONN_FLIP) {
-      if (j == fa) v = (int8_t)-v;
-    } else if (fa >= 0) {
-      if (j == fa) v = row[fb];
-      else if (j == fb) v = row[fa];
+      if (j == fa[k]) v = (int8_t)-v;
+    } else if (fa[k] >= 0) {
+      if (j == fa[k]) v = row[k][fb[k]];
+      else if (j == fb[k]) v = row[k][fa[k]];
     }
     return (float)v;
   };
-  float lr = 0.0f, li = 0.0f;
-  for (int h = lane; h < p.M; h += 64) {
-    float tr = p.b_re[h], ti = -p.b_im[h];
-    for (int j = 0; j < p.N; ++j) {
-      const float s = spin(j);
-      tr += p.w_re[(int64_t)j * p.M + h] * s;
-      ti -= p.w_im[(int64_t)j * p.M + h] * s;
+  // sites j0 .. j0 + RBM_NJ - 1 of the K configurations into LDS (zeros
+  // past the last site); only this wave reads them
+  auto stage = [&](int j0) {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int k = 0; k < K; ++k)
+      reinterpret_cast<float*>(s_spin[wave][k])[lane] = j0 + lane < p.N ? spin(k, j0 + lane) : 0.0f;
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+  };
+  float lr[K], li[K];
+#pragma unroll
+  for (int k = 0; k < K; ++k) lr[k] = li[k] = 0.0f;
+  if (p.N <= RBM_NJ) stage(0);
+  for (int h0 = 0; h0 < p.M; h0 += 64 * HPL) {
+    float tr[HPL][K], ti[HPL][K];
+    int h[HPL];
+#pragma unroll
+    for (int u = 0; u < HPL; ++u) {
+      h[u] = h0 + 64 * u + lane;
+      const int hc = h[u] < p.M ? h[u] : p.M - 1;
+#pragma unroll
+      for (int k = 0; k < K; ++k) {
+        tr[u][k] = p.b_re[hc];
+        ti[u][k] = -p.b_im[hc];
+      }
     }
-    lr += lncosh_re(tr, ti);
-    li += lncosh_im(tr, ti);
+    for (int j0 = 0; j0 < p.N; j0 += RBM_NJ) {
+      if (p.N > RBM_NJ) stage(j0);
+      const int jn = p.N - j0 < RBM_NJ ? p.N - j0 : RBM_NJ;
+      for (int j = 0; j < jn; j += 4) {
+        float wr[4][HPL], wi[4][HPL];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int64_t jj = j0 + (j + e < jn ? j + e : jn - 1);
+#pragma unroll
+          for (int u = 0; u < HPL; ++u) {
+            const int hc = h[u] < p.M ? h[u] : p.M - 1;
+            wr[e][u] = p.w_re[jj * p.M + hc];
+            wi[e][u] = p.w_im[jj * p.M + hc];
+          }
+        }
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+          const f32x4 s = s_spin[wave][k][j >> 2];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            if (j + e < jn) {
+#pragma unroll
+              for (int u = 0; u < HPL; ++u) {
+                tr[u][k] += wr[e][u] * s[e];
+                ti[u][k] -= wi[e][u] * s[e];
+              }
+            }
+          }
+        }
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < HPL; ++u) {
+      if (h[u] < p.M) {
+#pragma unroll 1
+        for (int k = 0; k < K; ++k) {
+          float r, i;
+          lncosh(tr[u][k], ti[u][k], r, i);
+          lr[k] += r;
+          li[k] += i;
+        }
+      }
+    }
   }
-  for (int j = lane; j < p.N; j += 64) {
-    const float s = spin(j);
-    lr += p.a_re[j] * s;
-    li -= p.a_im[j] * s;
-  }
-  lr = wave_sum(lr);
-  li = wave_sum(li);
-  if (lane == 0) {
-    out[2 * m] = lr;
-    out[2 * m + 1] = li;
+#pragma unroll
+  for (int k = 0; k < K; ++k) {
+    for (int j = lane; j < p.N; j += 64) {
+      const float s = spin(k, j);
+      lr[k] += p.a_re[j] * s;
+      li[k] -= p.a_im[j] * s;
+    }
+    const float sr = wave_sum(lr[k]), si = wave_sum(li[k]);
+    if (lane == 0 && m0 + k < M) {
+      out[2 * (m0 + k)] = sr;
+      out[2 * (m0 + k) + 1] = si;
+    }
   }
 }
 
@@ -489,9 +583,22 @@ int fk_rbm_log_psi(const float* w_re, const float* w_im, const float* b_re, cons
   FK_REQUIRE(w_re && w_im && b_re && b_im && a_re && a_im && spins && logpsi, "fk_rbm_log_psi: null pointer");
   FK_REQUIRE(!pairs || (conn_a && conn_b), "fk_rbm_log_psi: pairs need a connection table");
   RbmParams p{w_re, w_im, b_re, b_im, a_re, a_im, n_visible, n_hidden};
-  const int per_block = 4;
-  hipLaunchKernelGGL(rbm_log_psi_kernel, dim3(div_up(m_count, per_block)), dim3(64 * per_block), 0,
-                     (hipStream_t)stream, p, spins, pairs, m_dev, m_count, conn_kind, conn_a, conn_b, logpsi);
+  // eight configurations a wave once that still gives every CU eight waves
+  // (two per SIMD); fewer configurations go one to a wave.  Two hidden units
+  // per lane at a time keep the eight-configuration form at four waves per
+  // SIMD (four took 290 registers: one wave per SIMD).
+  auto launch = [&](auto kern, int k) {
+    hipLaunchKernelGGL(kern, dim3(div_up(m_count, (int64_t)k * RBM_WAVES)), dim3(64 * RBM_WAVES), 0,
+                       (hipStream_t)stream, p, spins, pairs, m_dev, m_count, conn_kind, conn_a, conn_b, logpsi);
+  };
+  const bool one = n_hidden <= 64;
+  if (m_count >= 64LL * device_cu_count()) {
+    if (one) launch(rbm_log_psi_kernel<8, 1>, 8);
+    else launch(rbm_log_psi_kernel<8, 2>, 8);
+  } else {
+    if (one) launch(rbm_log_psi_kernel<1, 1>, 1);
+    else launch(rbm_log_psi_kernel<1, 4>, 1);
+  }
   FK_CHECK_LAUNCH();
   return FK_OK;
 }

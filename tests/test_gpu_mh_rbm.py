@@ -230,3 +230,18 @@ def test_mh_injected_randomness_checked():
     sampler.randomness = (np.full((steps, 16), 16, np.int32), None, np.zeros((steps, 16)))
     with pytest.raises(ValueError):
         next(sampler)
+
+
+@pytest.mark.parametrize('n,alpha', [(1, 1), (5, 3), (64, 1), (67, 2), (130, 1)])
+def test_rbm_log_psi_many_configurations(rng, n, alpha):
+    """The eight-configurations-a-wave form (65,536 configurations, and seven
+    more so that the last wave is ragged) against one configuration a wave,
+    bit for bit, and against the oracle on a subset: sites past one LDS chunk
+    and hidden units that fill no wave."""
+    m = _rbm((n, 1), alpha, 0.3)
+    s = torch.as_tensor(rng.choice([-1, 0, 1], size=(65536 + 7, n)).astype(np.int8))
+    got = m.log_psi(s)
+    one = torch.cat([m.log_psi(s[:9]), m.log_psi(s[-9:])])
+    assert torch.equal(torch.cat([got[:9], got[-9:]]), one)
+    ref = _oracle_lp(m, s[-9:].numpy())
+    assert np.abs(got[-9:].real.cpu().numpy() - ref.real).max() / (np.abs(ref.real).max() + 1) < 1e-5
