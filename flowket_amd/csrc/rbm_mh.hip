@@ -40,10 +40,27 @@ __device__ __forceinline__ float lncosh_im(float x, float y) {
   return atan2f((e1 - e2) * sy, (e1 + e2) * cy);
 }
 
+// Sum over the wave, the butterfly v[l] + v[l ^ 32], then ^ 16, 8, 4, 2, 1, in
+// lane-permuting vector instructions: the halves and rows are exchanged by
+// permlane swaps, and after each step the sums repeat with the step's period,
+// so a rotation by 8 and by 4 within a row of 16 is the exchange with lane
+// ^ 8 and ^ 4.  (Six shuffles through LDS are a chain of about 400 cycles that
+// every Metropolis proposal waits for.)
+template <int CTRL>
+__device__ __forceinline__ float dpp_add(float v) {
+  return v + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, true));
+}
 __device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-  return v;
+  const u32x2 h = __builtin_bit_cast(u32x2, __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v),
+                                                                             false, false));
+  v = __uint_as_float(h[0]) + __uint_as_float(h[1]);
+  const u32x2 r = __builtin_bit_cast(u32x2, __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v),
+                                                                             false, false));
+  v = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+  v = dpp_add<0x128>(v);  // row_ror:8
+  v = dpp_add<0x124>(v);  // row_ror:4
+  v = dpp_add<0x4e>(v);   // quad_perm [2, 3, 0, 1]
+  return dpp_add<0xb1>(v);  // quad_perm [1, 0, 3, 2]
 }
 
 // lncosh(x + iy) with one exponential: of e^{x-|x|} and e^{-x-|x|} one is 1
@@ -231,119 +248,115 @@ struct MhArgs {
   int32_t* nonfinite;      // set to 1 when a proposal's log psi is not finite (or null)
 };
 
-template <int HPL>  // hidden units per lane (M <= 64 * HPL)
-__global__ __launch_bounds__(64) void mh_rbm_kernel(MhArgs a) {
-  const int lane = threadIdx.x;
+// One workgroup per chain, a wave per 64 hidden units (M <= 64 * NW), one
+// unit per lane.  A step is a serial chain -- theta', lncosh, the sum over
+// the units, the decision -- so it is latency that bounds a chain: all units
+// in one wave took the lncosh of four units per lane in turn.  1024 chains x
+// 319 exchange proposals of the 8x8 alpha-4 RBM: 921 us in one wave, 480 in
+// four with the proposals drawn 64 at a time (four waves that each drew every
+// proposal were no faster than one).
+// The waves exchange their units' terms through LDS (double-buffered, one
+// barrier a step); every wave then adds a lane's terms in unit order and
+// reduces over the lanes, so all reach the same decision, the one a single
+// wave would.
+template <int NW>
+__global__ __launch_bounds__(64 * NW) void mh_rbm_kernel(MhArgs a) {
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  __shared__ float s_part[2][NW][64];
   const int64_t ch = blockIdx.x;
   if (ch >= a.chains) return;
   const RbmParams& p = a.p;
   const int N = p.N, M = p.M;
   extern __shared__ int8_t s_state[];  // N spins of this chain
-  for (int j = lane; j < N; j += 64) s_state[j] = a.state[ch * N + j];
+  for (int j = threadIdx.x; j < N; j += 64 * NW) s_state[j] = a.state[ch * N + j];
   __syncthreads();
-  float tr[HPL], ti[HPL];
-#pragma unroll
-  for (int k = 0; k < HPL; ++k) {
-    const int h = lane + 64 * k;
-    float r = 0.0f, i = 0.0f;
-    if (h < M) {
-      r = p.b_re[h];
-      i = -p.b_im[h];
-      for (int j = 0; j < N; ++j) {
-        const float s = (float)s_state[j];
-        r += p.w_re[(int64_t)j * M + h] * s;
-        i -= p.w_im[(int64_t)j * M + h] * s;
-      }
+  const int h = (int)threadIdx.x;
+  const bool unit = h < M;
+  float tr = 0.0f, ti = 0.0f;
+  auto theta = [&]() {  // from the state
+    tr = p.b_re[h];
+    ti = -p.b_im[h];
+#pragma unroll 4
+    for (int j = 0; j < N; ++j) {
+      const float s = (float)s_state[j];
+      tr += p.w_re[(int64_t)j * M + h] * s;
+      ti -= p.w_im[(int64_t)j * M + h] * s;
     }
-    tr[k] = r;
-    ti[k] = i;
-  }
+  };
+  if (unit) theta();
   // Re lncosh(theta) of the current state, kept with theta (recomputed
   // only where theta changes)
-  float lc[HPL];
-#pragma unroll
-  for (int k = 0; k < HPL; ++k) lc[k] = (lane + 64 * k < M) ? lncosh_re(tr[k], ti[k]) : 0.0f;
+  float lc = unit ? lncosh_re(tr, ti) : 0.0f;
   const int64_t total = a.n_burn + a.n_record * (a.unused + 1);
   int64_t acc = 0;
-  // proposal of a step: sites (j2 = -1 for local moves) and uniform, from
-  // the injected arrays or the counter hash; it does not depend on earlier
-  // acceptances, so the next step's is drawn and its weight rows and
-  // visible biases are requested while the current step computes
-  int cj1 = 0, cj2 = -1;
-  double cu = 0.0;
-  float pw1r[HPL], pw1i[HPL], pw2r[HPL], pw2i[HPL];
-  float pa1 = 0.0f, pa2 = 0.0f;
-  auto prefetch = [&](int64_t st) {
-    int j1, j2 = -1;
-    double u;
+  // The proposal of a step: sites (j2 = -1 for local moves) and uniform, from
+  // the injected arrays or the counter hash.  It does not depend on earlier
+  // acceptances, so lane l draws that of step base + l, 64 steps at once
+  // (drawn by the whole wave for each step, the hash's 64-bit products were
+  // a third of a step), and the next step's weight rows and visible biases
+  // are requested while the current step computes.
+  int dj1 = 0, dj2 = -1;
+  double du = 0.0;
+  auto draw = [&](int64_t base) {
+    const int64_t st = base + lane;
+    if (st >= total) return;
+    int j1, mv = 0;
     if (a.r_u) {
       j1 = a.r_site[st * a.chains + ch];
-      u = a.r_u[st * a.chains + ch];
-      if (a.kind == 1) {
-        const int mv = a.r_move[st * a.chains + ch];
-        const int dy = mv / 3 - 1, dx = mv % 3 - 1;
-        const int y = j1 / a.W, x = j1 - (j1 / a.W) * a.W;
-        j2 = ((y + dy + a.H) % a.H) * a.W + ((x + dx + a.W) % a.W);
-      }
+      du = a.r_u[st * a.chains + ch];
+      if (a.kind == 1) mv = a.r_move[st * a.chains + ch];
     } else {
       j1 = (int)(u01(a.seed, ch, st, 0) * N);
       if (j1 >= N) j1 = N - 1;
-      u = u01(a.seed, ch, st, 1);
+      du = u01(a.seed, ch, st, 1);
       if (a.kind == 1) {
-        int mv = (int)(u01(a.seed, ch, st, 2) * 9.0);
+        mv = (int)(u01(a.seed, ch, st, 2) * 9.0);
         if (mv > 8) mv = 8;
-        const int dy = mv / 3 - 1, dx = mv % 3 - 1;
-        const int y = j1 / a.W, x = j1 - (j1 / a.W) * a.W;
-        j2 = ((y + dy + a.H) % a.H) * a.W + ((x + dx + a.W) % a.W);
       }
     }
-    cj1 = j1;
-    cj2 = j2;
-    cu = u;
-    const int jb = j2 >= 0 ? j2 : j1;
-#pragma unroll
-    for (int k = 0; k < HPL; ++k) {
-      const int h = lane + 64 * k;
-      pw1r[k] = h < M ? p.w_re[(int64_t)j1 * M + h] : 0.0f;
-      pw1i[k] = h < M ? p.w_im[(int64_t)j1 * M + h] : 0.0f;
-      pw2r[k] = h < M ? p.w_re[(int64_t)jb * M + h] : 0.0f;
-      pw2i[k] = h < M ? p.w_im[(int64_t)jb * M + h] : 0.0f;
+    dj1 = j1;
+    if (a.kind == 1) {
+      const int dy = mv / 3 - 1, dx = mv % 3 - 1;
+      const int y = j1 / a.W, x = j1 - (j1 / a.W) * a.W;
+      dj2 = ((y + dy + a.H) % a.H) * a.W + ((x + dx + a.W) % a.W);
     }
-    pa1 = p.a_re[j1];
+  };
+  int cj1 = 0, cj2 = -1;
+  double cu = 0.0;
+  float pw1r = 0.0f, pw1i = 0.0f, pw2r = 0.0f, pw2i = 0.0f;
+  float pa1 = 0.0f, pa2 = 0.0f;
+  auto prefetch = [&](int64_t st) {
+    const int l = (int)(st & 63);
+    if (l == 0) draw(st);
+    cj1 = __builtin_amdgcn_readlane(dj1, l);
+    cj2 = __builtin_amdgcn_readlane(dj2, l);
+    cu = __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(du), l),
+                          __builtin_amdgcn_readlane(__double2loint(du), l));
+    const int jb = cj2 >= 0 ? cj2 : cj1;
+    if (unit) {
+      pw1r = p.w_re[(int64_t)cj1 * M + h];
+      pw1i = p.w_im[(int64_t)cj1 * M + h];
+      pw2r = p.w_re[(int64_t)jb * M + h];
+      pw2i = p.w_im[(int64_t)jb * M + h];
+    }
+    pa1 = p.a_re[cj1];
     pa2 = p.a_re[jb];
   };
   if (total > 0) prefetch(0);
+  int buf = 0;
   for (int64_t step = 0; step < total; ++step) {
     if (step > 0 && (step & 255) == 0) {
       // refresh theta from the state (bounds the drift of the FP32
       // incremental updates)
-#pragma unroll
-      for (int k = 0; k < HPL; ++k) {
-        const int h = lane + 64 * k;
-        if (h < M) {
-          float r = p.b_re[h], i = -p.b_im[h];
-          for (int j = 0; j < N; ++j) {
-            const float s = (float)s_state[j];
-            r += p.w_re[(int64_t)j * M + h] * s;
-            i -= p.w_im[(int64_t)j * M + h] * s;
-          }
-          tr[k] = r;
-          ti[k] = i;
-          lc[k] = lncosh_re(r, i);
-        }
+      if (unit) {
+        theta();
+        lc = lncosh_re(tr, ti);
       }
     }
     // ---- proposal: drawn (and its weight rows requested) one step ahead
     const int j1 = cj1, j2 = cj2;
     const double u = cu;
-    float w1r[HPL], w1i[HPL], w2r[HPL], w2i[HPL];
-#pragma unroll
-    for (int k = 0; k < HPL; ++k) {
-      w1r[k] = pw1r[k];
-      w1i[k] = pw1i[k];
-      w2r[k] = pw2r[k];
-      w2i[k] = pw2i[k];
-    }
+    const float w1r = pw1r, w1i = pw1i, w2r = pw2r, w2i = pw2i;
     const float a1 = pa1, a2 = pa2;
     if (step + 1 < total) prefetch(step + 1);
     // sites that change: local -> j1; exchange -> j1 and j2 if they differ
@@ -355,46 +368,49 @@ __global__ __launch_bounds__(64) void mh_rbm_kernel(MhArgs a) {
       flip2 = flip1;
     }
     float dre = 0.0f;
-    float nr[HPL], ni[HPL], nl[HPL];
-    if (flip1) {
+    float nr = tr, ni = ti, nl = lc;
+    if (flip1) {  // uniform over the workgroup, as every branch of the step
       const float s2 = flip2 ? (float)s_state[j2] : 0.0f;
-#pragma unroll
-      for (int k = 0; k < HPL; ++k) {
-        const int h = lane + 64 * k;
-        nr[k] = tr[k];
-        ni[k] = ti[k];
-        if (h < M) {
-          nr[k] -= 2.0f * s1 * w1r[k];
-          ni[k] += 2.0f * s1 * w1i[k];
-          if (flip2) {
-            nr[k] -= 2.0f * s2 * w2r[k];
-            ni[k] += 2.0f * s2 * w2i[k];
-          }
-          nl[k] = lncosh_re(nr[k], ni[k]);
-          dre += nl[k] - lc[k];
+      if (unit) {
+        nr -= 2.0f * s1 * w1r;
+        ni += 2.0f * s1 * w1i;
+        if (flip2) {
+          nr -= 2.0f * s2 * w2r;
+          ni += 2.0f * s2 * w2i;
         }
+        nl = lncosh_re(nr, ni);
+      }
+      if constexpr (NW > 1) {
+        // (a wave writes a buffer again two exchanges later, after the barrier
+        // of the one between, which every reader of this one has reached)
+        float(*part)[64] = s_part[buf];
+        buf ^= 1;
+        part[wave][lane] = unit ? nl - lc : 0.0f;
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < NW; ++k) dre += part[k][lane];
+      } else {
+        dre += unit ? nl - lc : 0.0f;
       }
       dre = wave_sum(dre);
       dre += -2.0f * s1 * a1;
-      if (flip2) dre += -2.0f * (float)s_state[j2] * a2;
+      if (flip2) dre += -2.0f * s2 * a2;
     }
     // ---- acceptance (samplers/metropolis_hastings.py:106-110); a
     // candidate whose log psi is not finite is reported (the reference
     // raises, :103-105) and never accepted
     const bool finite = isfinite(dre);
-    if (!finite && a.nonfinite && lane == 0) a.nonfinite[0] = 1;
+    if (!finite && a.nonfinite && threadIdx.x == 0) a.nonfinite[0] = 1;
     const float lr = fminf(2.0f * dre, 0.0f);
     const bool accept = finite && (double)expf(lr) > u;
     if (accept) {
       if (flip1) {
-#pragma unroll
-        for (int k = 0; k < HPL; ++k) {
-          tr[k] = nr[k];
-          ti[k] = ni[k];
-          if (lane + 64 * k < M) lc[k] = nl[k];
-        }
-        __syncthreads();
-        if (lane == 0) {
+        tr = nr;
+        ti = ni;
+        lc = nl;
+        // every wave has read the state by the exchange's barrier above
+        if (NW == 1) __syncthreads();
+        if (threadIdx.x == 0) {
           if (flip2) {
             const int8_t t = s_state[j1];
             s_state[j1] = s_state[j2];
@@ -412,18 +428,26 @@ __global__ __launch_bounds__(64) void mh_rbm_kernel(MhArgs a) {
       const int64_t rs = step - a.n_burn;
       if ((rs + 1) % (a.unused + 1) == 0) {
         const int64_t rec = rs / (a.unused + 1);
-        for (int j = lane; j < N; j += 64) a.out[(ch * a.n_record + rec) * N + j] = s_state[j];
+        for (int j = threadIdx.x; j < N; j += 64 * NW) a.out[(ch * a.n_record + rec) * N + j] = s_state[j];
       }
     }
   }
-  for (int j = lane; j < N; j += 64) a.state[ch * N + j] = s_state[j];
-  // final log psi from theta
+  for (int j = threadIdx.x; j < N; j += 64 * NW) a.state[ch * N + j] = s_state[j];
+  if (threadIdx.x == 0) a.accepts[ch] = acc;
+  if (!a.logpsi) return;
+  // final log psi from theta, a lane's units in order
+  __shared__ float s_fin[NW][2][64];
+  if (unit) lncosh(tr, ti, tr, ti);
+  s_fin[wave][0][lane] = unit ? tr : 0.0f;
+  s_fin[wave][1][lane] = unit ? ti : 0.0f;
+  __syncthreads();
+  if (wave > 0) return;
   float lr = 0.0f, li = 0.0f;
 #pragma unroll
-  for (int k = 0; k < HPL; ++k) {
+  for (int k = 0; k < NW; ++k) {
     if (lane + 64 * k < M) {
-      lr += lncosh_re(tr[k], ti[k]);
-      li += lncosh_im(tr[k], ti[k]);
+      lr += s_fin[k][0][lane];
+      li += s_fin[k][1][lane];
     }
   }
   for (int j = lane; j < N; j += 64) {
@@ -434,11 +458,8 @@ __global__ __launch_bounds__(64) void mh_rbm_kernel(MhArgs a) {
   lr = wave_sum(lr);
   li = wave_sum(li);
   if (lane == 0) {
-    a.accepts[ch] = acc;
-    if (a.logpsi) {
-      a.logpsi[2 * ch] = lr;
-      a.logpsi[2 * ch + 1] = li;
-    }
+    a.logpsi[2 * ch] = lr;
+    a.logpsi[2 * ch + 1] = li;
   }
 }
 
@@ -636,17 +657,23 @@ int fk_mh_rbm(const float* w_re, const float* w_im, const float* b_re, const flo
   a.nonfinite = nonfinite;
   const size_t lds = (size_t)((n_visible + 15) & ~15);
   hipStream_t s = (hipStream_t)stream;
-  const int hpl = (n_hidden + 63) / 64;
-  if (hpl <= 1) hipLaunchKernelGGL(mh_rbm_kernel<1>, dim3((unsigned)chains), dim3(64), lds, s, a);
-  else if (hpl <= 2) hipLaunchKernelGGL(mh_rbm_kernel<2>, dim3((unsigned)chains), dim3(64), lds, s, a);
-  else if (hpl <= 4) hipLaunchKernelGGL(mh_rbm_kernel<4>, dim3((unsigned)chains), dim3(64), lds, s, a);
-  else if (hpl <= 8) hipLaunchKernelGGL(mh_rbm_kernel<8>, dim3((unsigned)chains), dim3(64), lds, s, a);
-  else {
-    set_error("fk_mh_rbm: at most 512 hidden units");
-    return FK_ERR_UNSUPPORTED;
-  }
-  FK_CHECK_LAUNCH();
-  return FK_OK;
+  const int waves = (n_hidden + 63) / 64;
+  auto launch = [&](auto kern, int nw) -> int {
+    // the state and the waves' exchange buffers together may pass the 64 KB
+    // that a launch gets unasked
+    if (lds > 48 * 1024)
+      FK_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                       (int)lds));
+    hipLaunchKernelGGL(kern, dim3((unsigned)chains), dim3(64 * nw), lds, s, a);
+    FK_CHECK_LAUNCH();
+    return FK_OK;
+  };
+  if (waves <= 1) return launch(mh_rbm_kernel<1>, 1);
+  if (waves <= 2) return launch(mh_rbm_kernel<2>, 2);
+  if (waves <= 4) return launch(mh_rbm_kernel<4>, 4);
+  if (waves <= 8) return launch(mh_rbm_kernel<8>, 8);
+  set_error("fk_mh_rbm: at most 512 hidden units");
+  return FK_ERR_UNSUPPORTED;
 }
 
 int fk_rbm_grad(const float* w_re, const float* w_im, const float* b_re, const float* b_im, const float* a_re,
