@@ -9,7 +9,62 @@
 
 namespace fk {
 
-// mean over rows of O_re and O_im (column means Obar)
+// Column kernels (o_mean, oh_times_u): a wave owns 64 x 4 consecutive columns
+// (one 16-byte load per lane, row and part) and the rows are dealt to the
+// waves of a workgroup in contiguous ranges, whose FP64 sums are added in
+// wave order through LDS.  HBM bound: with one thread per column group over
+// all rows, 215,492 columns were 3.3 waves per CU and 1024 rows of O streamed
+// at 3.2 TB/s; dealt, at 5.6 TB/s (558 -> 316 us; o_mean 573 -> 365).
+constexpr int COL_WAVES = 16;
+
+// Waves per workgroup: doubled until the grid has 16 waves per CU or a wave's
+// rows would be fewer than 16.
+int col_waves(int64_t groups, int64_t B) {
+  int w = 1;
+  while (w < COL_WAVES && groups * w < 16LL * device_cu_count() && B >= 32LL * w) w *= 2;
+  return w;
+}
+
+// Rows [first, last) of wave w of nw.
+__device__ __forceinline__ void wave_rows(int64_t B, int w, int nw, int64_t& first, int64_t& last) {
+  first = B * w / nw;
+  last = B * (w + 1) / nw;
+}
+
+// mean over rows of O_re and O_im (column means Obar), columns in fours
+__global__ __launch_bounds__(64 * COL_WAVES) void o_mean4_kernel(const f32x4* __restrict__ ore,
+                                                                 const f32x4* __restrict__ oim, int64_t B, int64_t P4,
+                                                                 f32x4* __restrict__ mre, f32x4* __restrict__ mim) {
+  extern __shared__ double red[];  // [waves][8][64]
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), nw = blockDim.x >> 6;
+  const int64_t t = (int64_t)blockIdx.x * 64 + lane;
+  int64_t b0, b1;
+  wave_rows(B, w, nw, b0, b1);
+  double acc[8] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+  if (t < P4) {
+#pragma unroll 4
+    for (int64_t b = b0; b < b1; ++b) {
+      const f32x4 x = ore[b * P4 + t], y = oim[b * P4 + t];
+#pragma unroll
+      for (int c = 0; c < 4; ++c) acc[c] += x[c], acc[4 + c] += y[c];
+    }
+  }
+#pragma unroll
+  for (int c = 0; c < 8; ++c) red[(w * 8 + c) * 64 + lane] = acc[c];
+  __syncthreads();
+  if (w > 0 || t >= P4) return;
+  f32x4 m[2];
+#pragma unroll
+  for (int c = 0; c < 8; ++c) {
+    double r = 0.0;
+    for (int k = 0; k < nw; ++k) r += red[(k * 8 + c) * 64 + lane];
+    m[c >> 2][c & 3] = (float)(r / (double)B);
+  }
+  mre[t] = m[0];
+  mim[t] = m[1];
+}
+
+// the same one column per thread (column counts that are no multiple of 4)
 __global__ void o_mean_kernel(const float* __restrict__ ore, const float* __restrict__ oim, int64_t B, int64_t P,
                               float* __restrict__ mre, float* __restrict__ mim) {
   const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -23,56 +78,94 @@ __global__ void o_mean_kernel(const float* __restrict__ ore, const float* __rest
   mim[k] = (float)(si / (double)B);
 }
 
+// Sum of a workgroup's values in a fixed tree; every thread gets it.  s: as
+// many doubles as threads (a power of two).
+__device__ __forceinline__ double block_sum(double x, double* s) {
+  __syncthreads();
+  s[threadIdx.x] = x;
+  __syncthreads();
+  for (int st = blockDim.x / 2; st > 0; st >>= 1) {
+    if ((int)threadIdx.x < st) s[threadIdx.x] += s[threadIdx.x + st];
+    __syncthreads();
+  }
+  return s[0];
+}
+
+// Dots leave DOT_BLOCKS partial sums; the kernels that need the dot add them
+// (block_sum of the first DOT_BLOCKS threads' loads: the same order in every
+// workgroup, so all agree bit for bit) instead of a launch of its own.
+constexpr int DOT_BLOCKS = 256;
+
+__device__ __forceinline__ double dot_total(const double* __restrict__ part, double* s) {
+  return block_sum((int)threadIdx.x < DOT_BLOCKS ? part[threadIdx.x] : 0.0, s);
+}
+
+// partials of a0 . b (out[0 .. DOT_BLOCKS)) and a1 . b (out[DOT_BLOCKS ..])
+__global__ __launch_bounds__(1024) void dot2_f64_kernel(const float* __restrict__ a0, const float* __restrict__ a1,
+                                                        const float* __restrict__ b, int64_t n,
+                                                        double* __restrict__ out) {
+  __shared__ double s[1024];
+  double acc0 = 0.0, acc1 = 0.0;
+  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
+    const double bi = b[i];
+    acc0 += (double)a0[i] * bi;
+    acc1 += (double)a1[i] * bi;
+  }
+  acc0 = block_sum(acc0, s);
+  acc1 = block_sum(acc1, s);
+  if (threadIdx.x == 0) {
+    out[blockIdx.x] = acc0;
+    out[DOT_BLOCKS + blockIdx.x] = acc1;
+  }
+}
+
 __global__ __launch_bounds__(1024) void dot_f64_kernel(const float* __restrict__ a, const float* __restrict__ b,
                                                        int64_t n, double* __restrict__ out) {
   __shared__ double s[1024];
   double acc = 0.0;
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
     acc += (double)a[i] * (double)b[i];
-  s[threadIdx.x] = acc;
-  __syncthreads();
-  for (int st = blockDim.x / 2; st > 0; st >>= 1) {
-    if ((int)threadIdx.x < st) s[threadIdx.x] += s[threadIdx.x + st];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) out[blockIdx.x] = s[0];
+  acc = block_sum(acc, s);
+  if (threadIdx.x == 0) out[blockIdx.x] = acc;
 }
 
-__global__ __launch_bounds__(256) void sum_f64_kernel(const double* __restrict__ in, int n, double* __restrict__ out) {
-  __shared__ double s[256];
-  double acc = 0.0;
-  for (int i = threadIdx.x; i < n; i += blockDim.x) acc += in[i];
-  s[threadIdx.x] = acc;
-  __syncthreads();
-  for (int st = blockDim.x / 2; st > 0; st >>= 1) {
-    if ((int)threadIdx.x < st) s[threadIdx.x] += s[threadIdx.x + st];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) out[0] = s[0];
+// out[k] = total of the k-th DOT_BLOCKS partials, k < gridDim.x
+__global__ __launch_bounds__(DOT_BLOCKS) void dot_totals_kernel(const double* __restrict__ part,
+                                                                double* __restrict__ out) {
+  __shared__ double s[DOT_BLOCKS];
+  const double x = dot_total(part + (int64_t)blockIdx.x * DOT_BLOCKS, s);
+  if (threadIdx.x == 0) out[blockIdx.x] = x;
 }
 
 // u_b = sum_k (O_bk - Obar_k) v_k = O_b.v - Obar.v (complex).  A workgroup
-// covers ROWS rows so each v_k is read once per ROWS rows; ov_c = Obar.v
-// (re, im) in FP64 is subtracted at the end.  With P a multiple of 4 the rows
-// are streamed as float4.
-constexpr int OV_ROWS = 4;
+// covers ROWS rows (each v_k read once for them) of column chunk blockIdx.y;
+// Obar.v in FP64, from its partial dots ov, is subtracted at the end.  With P
+// a multiple of 4 the rows are streamed as float4.  With one chunk u is
+// written here, with more the chunk's FP64 sums go to part ([chunk][row][2])
+// for ov_finish_kernel.
+constexpr int64_t OV_PARTS = 8192;  // (chunk, row) sums that the scratch holds
+
+template <int ROWS>
 __global__ __launch_bounds__(256) void o_times_v_kernel(const float* __restrict__ ore, const float* __restrict__ oim,
-                                                        const double* __restrict__ ov_c, const float* __restrict__ v,
-                                                        int64_t B, int64_t P, float* __restrict__ u) {
-  __shared__ double s_r[OV_ROWS][256], s_i[OV_ROWS][256];
-  const int64_t b0 = (int64_t)blockIdx.x * OV_ROWS;
-  double dr[OV_ROWS], di[OV_ROWS];
-  float ar[OV_ROWS], ai[OV_ROWS];
+                                                        const double* __restrict__ ov, const float* __restrict__ v,
+                                                        int64_t B, int64_t P, double* __restrict__ part,
+                                                        float* __restrict__ u) {
+  __shared__ double red[256];
+  const int64_t b0 = (int64_t)blockIdx.x * ROWS;
+  double dr[ROWS], di[ROWS];
+  float ar[ROWS], ai[ROWS];
 #pragma unroll
-  for (int r = 0; r < OV_ROWS; ++r) dr[r] = di[r] = 0.0, ar[r] = ai[r] = 0.0f;
+  for (int r = 0; r < ROWS; ++r) dr[r] = di[r] = 0.0, ar[r] = ai[r] = 0.0f;
   int cnt = 0;
   if ((P & 3) == 0) {
     const int64_t P4 = P >> 2;
+    const int64_t k1 = P4 * (blockIdx.y + 1) / gridDim.y;
     const f32x4* v4 = reinterpret_cast<const f32x4*>(v);
-    for (int64_t k = threadIdx.x; k < P4; k += blockDim.x) {
+#pragma unroll 4
+    for (int64_t k = P4 * blockIdx.y / gridDim.y + threadIdx.x; k < k1; k += 256) {
       const f32x4 vk = v4[k];
 #pragma unroll
-      for (int r = 0; r < OV_ROWS; ++r) {
+      for (int r = 0; r < ROWS; ++r) {
         if (b0 + r < B) {
           const f32x4 x = reinterpret_cast<const f32x4*>(ore + (b0 + r) * P)[k];
           const f32x4 y = reinterpret_cast<const f32x4*>(oim + (b0 + r) * P)[k];
@@ -82,15 +175,16 @@ __global__ __launch_bounds__(256) void o_times_v_kernel(const float* __restrict_
       }
       if (++cnt == 16) {  // fold fp32 partials into fp64 every 64 terms
 #pragma unroll
-        for (int r = 0; r < OV_ROWS; ++r) dr[r] += ar[r], di[r] += ai[r], ar[r] = ai[r] = 0.0f;
+        for (int r = 0; r < ROWS; ++r) dr[r] += ar[r], di[r] += ai[r], ar[r] = ai[r] = 0.0f;
         cnt = 0;
       }
     }
   } else {
-    for (int64_t k = threadIdx.x; k < P; k += blockDim.x) {
+    const int64_t k1 = P * (blockIdx.y + 1) / gridDim.y;
+    for (int64_t k = P * blockIdx.y / gridDim.y + threadIdx.x; k < k1; k += 256) {
       const float vk = v[k];
 #pragma unroll
-      for (int r = 0; r < OV_ROWS; ++r) {
+      for (int r = 0; r < ROWS; ++r) {
         if (b0 + r < B) {
           ar[r] += ore[(b0 + r) * P + k] * vk;
           ai[r] += oim[(b0 + r) * P + k] * vk;
@@ -98,32 +192,46 @@ __global__ __launch_bounds__(256) void o_times_v_kernel(const float* __restrict_
       }
       if (++cnt == 64) {
 #pragma unroll
-        for (int r = 0; r < OV_ROWS; ++r) dr[r] += ar[r], di[r] += ai[r], ar[r] = ai[r] = 0.0f;
+        for (int r = 0; r < ROWS; ++r) dr[r] += ar[r], di[r] += ai[r], ar[r] = ai[r] = 0.0f;
         cnt = 0;
       }
     }
   }
-#pragma unroll
-  for (int r = 0; r < OV_ROWS; ++r) {
-    s_r[r][threadIdx.x] = dr[r] + ar[r];
-    s_i[r][threadIdx.x] = di[r] + ai[r];
+  double ovr = 0.0, ovi = 0.0;
+  if (!part) {
+    ovr = dot_total(ov, red);
+    ovi = dot_total(ov + DOT_BLOCKS, red);
   }
-  __syncthreads();
-  for (int s = blockDim.x / 2; s > 0; s >>= 1) {
-    if ((int)threadIdx.x < s) {
 #pragma unroll
-      for (int r = 0; r < OV_ROWS; ++r) {
-        s_r[r][threadIdx.x] += s_r[r][threadIdx.x + s];
-        s_i[r][threadIdx.x] += s_i[r][threadIdx.x + s];
+  for (int r = 0; r < ROWS; ++r) {
+    const double sr = block_sum(dr[r] + ar[r], red), si = block_sum(di[r] + ai[r], red);
+    if (threadIdx.x == 0 && b0 + r < B) {
+      if (part) {
+        part[((int64_t)blockIdx.y * B + b0 + r) * 2] = sr;
+        part[((int64_t)blockIdx.y * B + b0 + r) * 2 + 1] = si;
+      } else {
+        u[2 * (b0 + r)] = (float)(sr - ovr);
+        u[2 * (b0 + r) + 1] = (float)(si - ovi);
       }
     }
-    __syncthreads();
   }
-  if ((int)threadIdx.x < OV_ROWS && b0 + threadIdx.x < B) {
-    const int r = threadIdx.x;
-    u[2 * (b0 + r)] = (float)(s_r[r][0] - ov_c[0]);
-    u[2 * (b0 + r) + 1] = (float)(s_i[r][0] - ov_c[1]);
+}
+
+// u of the rows from their chunks' sums, added in chunk order.
+__global__ __launch_bounds__(256) void ov_finish_kernel(const double* __restrict__ part, int64_t chunks,
+                                                        const double* __restrict__ ov, int64_t B,
+                                                        float* __restrict__ u) {
+  __shared__ double red[256];
+  const double ovr = dot_total(ov, red), ovi = dot_total(ov + DOT_BLOCKS, red);
+  const int64_t b = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (b >= B) return;
+  double r = 0.0, i = 0.0;
+  for (int64_t c = 0; c < chunks; ++c) {
+    r += part[(c * B + b) * 2];
+    i += part[(c * B + b) * 2 + 1];
   }
+  u[2 * b] = (float)(r - ovr);
+  u[2 * b + 1] = (float)(i - ovi);
 }
 
 __global__ __launch_bounds__(1024) void sum_u_kernel(const float* __restrict__ u, int64_t B, double* __restrict__ out) {
@@ -157,42 +265,49 @@ __global__ void center_pairs_kernel(float* __restrict__ u, int64_t B, const doub
   u[2 * b + 1] = (float)((double)u[2 * b + 1] - sums[1] / (double)B);
 }
 
-// out_k = scale * Re[sum_b conj(O_bk - Obar_k) u_b] + shift * v_k; each
-// thread owns 4 consecutive columns (float4 rows) when P is a multiple of 4.
+// out_k = scale * Re[sum_b conj(O_bk - Obar_k) u_b] + shift * v_k, columns in
+// fours (a column kernel, see o_mean4_kernel); FP32 over 64 rows, then FP64.
+__global__ __launch_bounds__(64 * COL_WAVES) void oh_times_u4_kernel(
+    const f32x4* __restrict__ ore, const f32x4* __restrict__ oim, const float* __restrict__ mre,
+    const float* __restrict__ mim, const float* __restrict__ u, const double* __restrict__ usum, int64_t B, int64_t P4,
+    double scale, double shift, const float* __restrict__ v, float* __restrict__ out) {
+  extern __shared__ double red[];  // [waves][4][64]
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), nw = blockDim.x >> 6;
+  const int64_t t = (int64_t)blockIdx.x * 64 + lane;
+  int64_t b0, b1;
+  wave_rows(B, w, nw, b0, b1);
+  double acc[4] = {0.0, 0.0, 0.0, 0.0};
+  if (t < P4) {
+    for (int64_t c0 = b0; c0 < b1; c0 += 64) {
+      const int64_t c1 = c0 + 64 < b1 ? c0 + 64 : b1;
+      f32x4 part = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 8
+      for (int64_t b = c0; b < c1; ++b) part += ore[b * P4 + t] * u[2 * b] + oim[b * P4 + t] * u[2 * b + 1];
+#pragma unroll
+      for (int c = 0; c < 4; ++c) acc[c] += part[c];
+    }
+  }
+#pragma unroll
+  for (int c = 0; c < 4; ++c) red[(w * 4 + c) * 64 + lane] = acc[c];
+  __syncthreads();
+  if (w > 0 || t >= P4) return;
+#pragma unroll
+  for (int c = 0; c < 4; ++c) {
+    double r = 0.0;
+    for (int q = 0; q < nw; ++q) r += red[(q * 4 + c) * 64 + lane];
+    const int64_t k = 4 * t + c;
+    r = scale * (r - ((double)mre[k] * usum[0] + (double)mim[k] * usum[1]));
+    if (v) r += shift * (double)v[k];
+    out[k] = (float)r;
+  }
+}
+
+// the same one column per thread (column counts that are no multiple of 4)
 __global__ void oh_times_u_kernel(const float* __restrict__ ore, const float* __restrict__ oim,
                                   const float* __restrict__ mre, const float* __restrict__ mim,
                                   const float* __restrict__ u, const double* __restrict__ usum, int64_t B, int64_t P,
                                   double scale, double shift, const float* __restrict__ v, float* __restrict__ out) {
-  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if ((P & 3) == 0) {
-    const int64_t P4 = P >> 2;
-    if (t >= P4) return;
-    double acc[4] = {0.0, 0.0, 0.0, 0.0};
-    f32x4 part = {0.f, 0.f, 0.f, 0.f};
-    int cnt = 0;
-#pragma unroll 8
-    for (int64_t b = 0; b < B; ++b) {
-      const f32x4 x = reinterpret_cast<const f32x4*>(ore + b * P)[t];
-      const f32x4 y = reinterpret_cast<const f32x4*>(oim + b * P)[t];
-      const float ur = u[2 * b], ui = u[2 * b + 1];
-      part += x * ur + y * ui;
-      if (++cnt == 64) {
-        acc[0] += part.x, acc[1] += part.y, acc[2] += part.z, acc[3] += part.w;
-        part = f32x4{0.f, 0.f, 0.f, 0.f};
-        cnt = 0;
-      }
-    }
-    acc[0] += part.x, acc[1] += part.y, acc[2] += part.z, acc[3] += part.w;
-#pragma unroll
-    for (int c = 0; c < 4; ++c) {
-      const int64_t k = 4 * t + c;
-      double r = scale * (acc[c] - ((double)mre[k] * usum[0] + (double)mim[k] * usum[1]));
-      if (v) r += shift * (double)v[k];
-      out[k] = (float)r;
-    }
-    return;
-  }
-  const int64_t k = t;
+  const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (k >= P) return;
   double acc = 0.0;
   float part = 0.0f;
@@ -410,24 +525,43 @@ __global__ void cg_init_scalars_kernel(double* st, double tol, double max_iter) 
   st[CG_DONE] = (max_iter <= 0.0 || !((double)nb > st[CG_TOL])) ? 1.0 : 0.0;
 }
 
-__global__ void cg_update_xr_kernel(const double* __restrict__ st, const float* __restrict__ p,
-                                    const float* __restrict__ z, float* __restrict__ x, float* __restrict__ r,
-                                    int64_t n) {
-  if (st[CG_DONE] != 0.0) return;
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const double alpha = st[CG_GAMMA] / st[CG_PZ];
-  x[i] = (float)((double)x[i] + alpha * (double)p[i]);
-  r[i] = (float)((double)r[i] - alpha * (double)z[i]);
+// x += alpha p, r -= alpha z with alpha = gamma / (p . z) from the partial
+// dots pz; the partial dots of the new r go to rr.  DOT_BLOCKS workgroups.
+__global__ __launch_bounds__(1024) void cg_update_xr_kernel(double* __restrict__ st, const double* __restrict__ pz,
+                                                            const float* __restrict__ p, const float* __restrict__ z,
+                                                            float* __restrict__ x, float* __restrict__ r, int64_t n,
+                                                            double* __restrict__ rr) {
+  __shared__ double s[1024];
+  const bool done = st[CG_DONE] != 0.0;
+  const double pdz = dot_total(pz, s);
+  if (blockIdx.x == 0 && threadIdx.x == 0) st[CG_PZ] = pdz;
+  const double alpha = st[CG_GAMMA] / pdz;
+  double acc = 0.0;
+  for (int64_t i = (int64_t)blockIdx.x * 1024 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 1024) {
+    float ri = r[i];
+    if (!done) {
+      x[i] = (float)((double)x[i] + alpha * (double)p[i]);
+      ri = (float)((double)ri - alpha * (double)z[i]);
+      r[i] = ri;
+    }
+    acc += (double)ri * (double)ri;
+  }
+  acc = block_sum(acc, s);
+  if (threadIdx.x == 0) rr[blockIdx.x] = acc;
 }
 
-__global__ void cg_update_p_kernel(const double* __restrict__ st, const float* __restrict__ r, float* __restrict__ p,
-                                   int64_t n) {
+// p = r + beta p with beta = r . r / gamma, and r . r from its partials; the
+// state itself is advanced by cg_finish_step_kernel, once all have read it.
+__global__ __launch_bounds__(1024) void cg_update_p_kernel(double* __restrict__ st, const double* __restrict__ rr,
+                                                           const float* __restrict__ r, float* __restrict__ p,
+                                                           int64_t n) {
+  __shared__ double s[1024];
+  const double gnew = dot_total(rr, s);
+  if (blockIdx.x == 0 && threadIdx.x == 0) st[CG_GNEW] = gnew;
   if (st[CG_DONE] != 0.0) return;
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const double beta = st[CG_GNEW] / st[CG_GAMMA];
-  p[i] = (float)((double)r[i] + beta * (double)p[i]);
+  const double beta = gnew / st[CG_GAMMA];
+  for (int64_t i = (int64_t)blockIdx.x * 1024 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 1024)
+    p[i] = (float)((double)r[i] + beta * (double)p[i]);
 }
 
 __global__ void cg_finish_step_kernel(double* st) {
@@ -479,8 +613,16 @@ int fk_o_mean(const float* o_re, const float* o_im, int64_t batch, int64_t n_par
               void* stream) {
   FK_REQUIRE(o_re && o_im && mean_re && mean_im, "fk_o_mean: null pointer");
   FK_REQUIRE(batch > 0 && n_params > 0, "fk_o_mean: empty");
-  hipLaunchKernelGGL(o_mean_kernel, dim3(div_up(n_params, 256)), dim3(256), 0, (hipStream_t)stream, o_re, o_im, batch,
-                     n_params, mean_re, mean_im);
+  if ((n_params & 3) || (((uintptr_t)o_re | (uintptr_t)o_im | (uintptr_t)mean_re | (uintptr_t)mean_im) & 15)) {
+    hipLaunchKernelGGL(o_mean_kernel, dim3(div_up(n_params, 256)), dim3(256), 0, (hipStream_t)stream, o_re, o_im,
+                       batch, n_params, mean_re, mean_im);
+  } else {
+    const int64_t p4 = n_params / 4;
+    const int nw = col_waves(div_up(p4, 64), batch);
+    hipLaunchKernelGGL(o_mean4_kernel, dim3(div_up(p4, 64)), dim3(64 * nw), (size_t)nw * 8 * 64 * sizeof(double),
+                       (hipStream_t)stream, reinterpret_cast<const f32x4*>(o_re), reinterpret_cast<const f32x4*>(o_im),
+                       batch, p4, reinterpret_cast<f32x4*>(mean_re), reinterpret_cast<f32x4*>(mean_im));
+  }
   FK_CHECK_LAUNCH();
   return FK_OK;
 }
@@ -490,18 +632,34 @@ int fk_o_times_v(const float* o_re, const float* o_im, const float* mean_re, con
   FK_REQUIRE(o_re && o_im && mean_re && mean_im && v && u && scratch, "fk_o_times_v: null pointer");
   FK_REQUIRE(batch > 0 && n_params > 0, "fk_o_times_v: bad sizes");
   hipStream_t s = (hipStream_t)stream;
-  // scratch: [0..255] partials, [256] Obar_re.v, [257] Obar_im.v
-  hipLaunchKernelGGL(dot_f64_kernel, dim3(256), dim3(1024), 0, s, mean_re, v, n_params, scratch);
+  // scratch: [0, 2 DOT_BLOCKS) the partials of Obar.v, then the chunks' sums
+  hipLaunchKernelGGL(dot2_f64_kernel, dim3(DOT_BLOCKS), dim3(1024), 0, s, mean_re, mean_im, v, n_params, scratch);
   FK_CHECK_LAUNCH();
-  hipLaunchKernelGGL(sum_f64_kernel, dim3(1), dim3(256), 0, s, scratch, 256, scratch + 256);
+  // Four rows a workgroup where that still gives every CU four workgroups;
+  // else one row, and where even the rows are too few, column chunks of at
+  // least 8 KB (1024 rows of 215,492 columns: 788 us in groups of four rows,
+  // four waves per CU; 299 us, 5.9 TB/s, one row each).
+  const int64_t want = 4LL * device_cu_count();
+  const int64_t rows = batch >= 4 * want ? 4 : 1;
+  int64_t chunks = 1;
+  if (batch < want) {
+    chunks = (want + batch - 1) / batch;
+    if (chunks > n_params / 2048) chunks = n_params / 2048;
+    if (chunks * batch > OV_PARTS) chunks = OV_PARTS / batch;
+    if (chunks < 1) chunks = 1;
+  }
+  double* part = chunks > 1 ? scratch + 2 * DOT_BLOCKS : nullptr;
+  if (rows == 4)
+    hipLaunchKernelGGL(o_times_v_kernel<4>, dim3(div_up(batch, 4)), dim3(256), 0, s, o_re, o_im, scratch, v, batch,
+                       n_params, part, u);
+  else
+    hipLaunchKernelGGL(o_times_v_kernel<1>, dim3((unsigned)batch, (unsigned)chunks), dim3(256), 0, s, o_re, o_im,
+                       scratch, v, batch, n_params, part, u);
   FK_CHECK_LAUNCH();
-  hipLaunchKernelGGL(dot_f64_kernel, dim3(256), dim3(1024), 0, s, mean_im, v, n_params, scratch);
-  FK_CHECK_LAUNCH();
-  hipLaunchKernelGGL(sum_f64_kernel, dim3(1), dim3(256), 0, s, scratch, 256, scratch + 257);
-  FK_CHECK_LAUNCH();
-  hipLaunchKernelGGL(o_times_v_kernel, dim3(div_up(batch, OV_ROWS)), dim3(256), 0, s, o_re, o_im, scratch + 256, v,
-                     batch, n_params, u);
-  FK_CHECK_LAUNCH();
+  if (part) {
+    hipLaunchKernelGGL(ov_finish_kernel, dim3(div_up(batch, 256)), dim3(256), 0, s, part, chunks, scratch, batch, u);
+    FK_CHECK_LAUNCH();
+  }
   return FK_OK;
 }
 
@@ -513,14 +671,21 @@ int fk_oh_times_u(const float* o_re, const float* o_im, const float* mean_re, co
   hipStream_t s = (hipStream_t)stream;
   hipLaunchKernelGGL(sum_u_kernel, dim3(1), dim3(1024), 0, s, u, batch, scratch2);
   FK_CHECK_LAUNCH();
-  const int64_t cols = (n_params & 3) == 0 ? n_params / 4 : n_params;
-  hipLaunchKernelGGL(oh_times_u_kernel, dim3(div_up(cols, 256)), dim3(256), 0, s, o_re, o_im, mean_re, mean_im, u,
-                     scratch2, batch, n_params, scale, shift, v, out);
+  if (n_params & 3) {
+    hipLaunchKernelGGL(oh_times_u_kernel, dim3(div_up(n_params, 256)), dim3(256), 0, s, o_re, o_im, mean_re, mean_im, u,
+                       scratch2, batch, n_params, scale, shift, v, out);
+  } else {
+    const int64_t p4 = n_params / 4;
+    const int nw = col_waves(div_up(p4, 64), batch);
+    hipLaunchKernelGGL(oh_times_u4_kernel, dim3(div_up(p4, 64)), dim3(64 * nw), (size_t)nw * 4 * 64 * sizeof(double), s,
+                       reinterpret_cast<const f32x4*>(o_re), reinterpret_cast<const f32x4*>(o_im), mean_re, mean_im, u,
+                       scratch2, batch, p4, scale, shift, v, out);
+  }
   FK_CHECK_LAUNCH();
   return FK_OK;
 }
 
-int64_t fk_sr_scratch_doubles(void) { return 260; }
+int64_t fk_sr_scratch_doubles(void) { return 2 * DOT_BLOCKS + 2 * OV_PARTS; }
 
 int64_t fk_sr_matvec_workspace_bytes(int64_t batch, int64_t n_params) {
   (void)batch;
@@ -543,18 +708,17 @@ int fk_sr_matvec(const float* o_re, const float* o_im, const float* mean_re, con
              (long long)fk_sr_matvec_workspace_bytes(batch, n_params));
   FK_REQUIRE(((uintptr_t)workspace & 15) == 0, "fk_sr_matvec: workspace must be 16-byte aligned");
   hipStream_t s = (hipStream_t)stream;
-  // scratch: [0..255] dot partials, [256..257] Obar.v, [258..259] sum_b u_b
-  for (int part = 0; part < 2; ++part) {
-    hipLaunchKernelGGL(dot_f64_kernel, dim3(256), dim3(1024), 0, s, part ? mean_im : mean_re, v, n_params, scratch);
-    FK_CHECK_LAUNCH();
-    hipLaunchKernelGGL(sum_f64_kernel, dim3(1), dim3(256), 0, s, scratch, 256, scratch + 256 + part);
-    FK_CHECK_LAUNCH();
-  }
+  // scratch: the partials of Obar.v, then Obar.v and sum_b u_b
+  double* sums = scratch + 2 * DOT_BLOCKS;
+  hipLaunchKernelGGL(dot2_f64_kernel, dim3(DOT_BLOCKS), dim3(1024), 0, s, mean_re, mean_im, v, n_params, scratch);
+  FK_CHECK_LAUNCH();
+  hipLaunchKernelGGL(dot_totals_kernel, dim3(2), dim3(DOT_BLOCKS), 0, s, scratch, sums);
+  FK_CHECK_LAUNCH();
   SvArgs a{};
   a.ore = o_re;
   a.oim = o_im;
   a.v = v;
-  a.ov_c = scratch + 256;
+  a.ov_c = sums;
   a.part = reinterpret_cast<double*>(workspace);
   a.acc = a.part + 2 * SV_MAXR * SV_NA * 2;
   a.u = u;
@@ -571,10 +735,10 @@ int fk_sr_matvec(const float* o_re, const float* o_im, const float* mean_re, con
     hipLaunchKernelGGL(sv_rows_kernel, dim3(grid), dim3(SV_T), 0, s, a);
     FK_CHECK_LAUNCH();
   }
-  hipLaunchKernelGGL(sum_u_kernel, dim3(1), dim3(1024), 0, s, u, batch, scratch + 258);
+  hipLaunchKernelGGL(sum_u_kernel, dim3(1), dim3(1024), 0, s, u, batch, sums + 2);
   FK_CHECK_LAUNCH();
   hipLaunchKernelGGL(sv_finish_kernel, dim3(div_up(n_params, 256)), dim3(256), 0, s, a.acc, mean_re, mean_im,
-                     scratch + 258, n_params, scale, shift, v, out);
+                     sums + 2, n_params, scale, shift, v, out);
   FK_CHECK_LAUNCH();
   return FK_OK;
 }
@@ -582,10 +746,9 @@ int fk_sr_matvec(const float* o_re, const float* o_im, const float* mean_re, con
 int fk_dot_f64(const float* a, const float* b, int64_t n, double* scratch, double* out, void* stream) {
   FK_REQUIRE(a && b && scratch && out, "fk_dot_f64: null pointer");
   hipStream_t s = (hipStream_t)stream;
-  const int blocks = 256;
-  hipLaunchKernelGGL(dot_f64_kernel, dim3(blocks), dim3(1024), 0, s, a, b, n, scratch);
+  hipLaunchKernelGGL(dot_f64_kernel, dim3(DOT_BLOCKS), dim3(1024), 0, s, a, b, n, scratch);
   FK_CHECK_LAUNCH();
-  hipLaunchKernelGGL(sum_f64_kernel, dim3(1), dim3(256), 0, s, scratch, blocks, out);
+  hipLaunchKernelGGL(dot_totals_kernel, dim3(1), dim3(DOT_BLOCKS), 0, s, scratch, out);
   FK_CHECK_LAUNCH();
   return FK_OK;
 }
@@ -609,13 +772,13 @@ int fk_cg_step(float* x, float* r, float* p, const float* z, int64_t n, double* 
                void* stream) {
   FK_REQUIRE(x && r && p && z && state && scratch && n > 0, "fk_cg_step: bad arguments");
   hipStream_t s = (hipStream_t)stream;
-  int rc = fk_dot_f64(p, z, n, scratch, state + CG_PZ, stream);
-  if (rc != FK_OK) return rc;
-  hipLaunchKernelGGL(cg_update_xr_kernel, dim3(div_up(n, 256)), dim3(256), 0, s, state, p, z, x, r, n);
+  // four launches: each dot's total is taken by the kernel that needs it
+  hipLaunchKernelGGL(dot_f64_kernel, dim3(DOT_BLOCKS), dim3(1024), 0, s, p, z, n, scratch);
   FK_CHECK_LAUNCH();
-  rc = fk_dot_f64(r, r, n, scratch, state + CG_GNEW, stream);
-  if (rc != FK_OK) return rc;
-  hipLaunchKernelGGL(cg_update_p_kernel, dim3(div_up(n, 256)), dim3(256), 0, s, state, r, p, n);
+  hipLaunchKernelGGL(cg_update_xr_kernel, dim3(DOT_BLOCKS), dim3(1024), 0, s, state, scratch, p, z, x, r, n,
+                     scratch + DOT_BLOCKS);
+  FK_CHECK_LAUNCH();
+  hipLaunchKernelGGL(cg_update_p_kernel, dim3(DOT_BLOCKS), dim3(1024), 0, s, state, scratch + DOT_BLOCKS, r, p, n);
   FK_CHECK_LAUNCH();
   hipLaunchKernelGGL(cg_finish_step_kernel, dim3(1), dim3(1), 0, s, state);
   FK_CHECK_LAUNCH();

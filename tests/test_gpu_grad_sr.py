@@ -309,3 +309,38 @@ def test_mini_batch_loss_gradients_add_up_to_the_energy_gradient():
     assert sgd.iterations == 1
     # (params are FP32: the difference carries their rounding, a few 1e-8)
     assert torch.allclose(before - m.params, 1e-3 * acc, rtol=1e-4, atol=2e-7)
+
+
+@pytest.mark.parametrize('B,P', [(1, 4), (3, 260), (33, 8196), (255, 4100), (1023, 2052), (4099, 516), (7, 8191)])
+def test_sr_products_row_and_chunk_splits(B, P):
+    """Column means, (O-Obar) v and Re[(O-Obar)^H u] where the splits change:
+    column chunks (few rows), one and four rows a workgroup, rows dealt to 1 to
+    16 waves, and a column count that is no multiple of 4.  Tolerance: O, v
+    and u are N(0, 1); products are FP32 over 64 terms (sqrt(64) 2^-24 each,
+    random), then FP64: 1e-6 of the result's norm, and 1e-6 of a mean's."""
+    from flowket_amd import _lib
+    gen = torch.Generator(device='cuda').manual_seed(B * 7 + P)
+    ore, oim = [torch.randn((B, P), device='cuda', generator=gen) for _ in range(2)]
+    v = torch.randn(P, device='cuda', generator=gen)
+    mre, mim = torch.empty(P, device='cuda'), torch.empty(P, device='cuda')
+    s = _lib.stream_ptr()
+    _lib.call('fk_o_mean', _lib.ptr(ore), _lib.ptr(oim), B, P, _lib.ptr(mre), _lib.ptr(mim), s)
+    scratch = torch.empty(int(_lib.load().fk_sr_scratch_doubles()), dtype=torch.float64, device='cuda')
+    u = torch.empty((B, 2), device='cuda')
+    _lib.call('fk_o_times_v', _lib.ptr(ore), _lib.ptr(oim), _lib.ptr(mre), _lib.ptr(mim), _lib.ptr(v), B, P,
+              _lib.ptr(u), _lib.ptr(scratch), s)
+    w = torch.randn((B, 2), device='cuda', generator=gen)
+    out = torch.empty(P, device='cuda')
+    _lib.call('fk_oh_times_u', _lib.ptr(ore), _lib.ptr(oim), _lib.ptr(mre), _lib.ptr(mim), _lib.ptr(w), B, P, 0.5, 2.0,
+              _lib.ptr(v), _lib.ptr(out), _lib.ptr(scratch), s)
+    o = torch.complex(ore.double(), oim.double())
+    mean = o.mean(dim=0)
+    got = torch.complex(mre.double(), mim.double())
+    assert ((got - mean).norm() / mean.norm()).item() < 1e-6
+    oc = o - torch.complex(mre.double(), mim.double())
+    scale = (o.abs() ** 2 @ (v.double() ** 2)).sqrt()  # the size of the sums before Obar.v is taken off
+    ref = oc @ v.double().to(oc.dtype)
+    assert ((torch.view_as_complex(u.double()) - ref).abs() / scale).max().item() < 1e-6
+    refh = 0.5 * (oc.conj().T @ torch.view_as_complex(w.double())).real + 2.0 * v.double()
+    scale = 0.5 * (o.abs() ** 2).sum(dim=0).sqrt() * w.abs().max().double() + 2.0 * v.abs().double()
+    assert ((out.double() - refh).abs() / scale).max().item() < 1e-6
