@@ -16,123 +16,16 @@
 // 16 samples is (3*nb-2) lattices of 16 x C values.  The arithmetic, the
 // accumulation order and the roundings are those of the fused forward kernel,
 // so the draws equal the plain sampler's draws given the same uniforms.
-#include "fk_common.h"
-#include "convar_layout.h"
-#include "convar_dev.h"
+//
+// Most networks take the workgroup-per-tile kernel of fast_sampler_mw.hip;
+// this one draws from those that it does not take (fast_mw_supported).  Its
+// whole-row form stays for two-block networks on rows of at most VROW_MAX
+// pixels (10x10, 1024 samples: 0.32 ms against 0.48 without it).
+#include "fast_sampler.h"
 
 #include <type_traits>
 
 namespace fk {
-
-// Per-lane data of one pixel of a C-channel tensor for 16 samples: MT quads
-// of 4 channels (channels 16*mt + 4*g + r for lane group g) in M-tile order.
-template <int PREC, int C>
-struct LaneData;
-
-// 16-bit precisions (bf16, fp16): 8 bytes per quad
-template <int PREC, int C>
-struct LaneData {
-  static constexpr int MT = C / 16;
-  static constexpr int LB = MT * 8;  // bytes per lane
-  uint2 q[MT];
-  __device__ __forceinline__ void load(const uint8_t* p) {
-#pragma unroll
-    for (int k = 0; k < MT / 2; ++k) {
-      const uint4 v = *reinterpret_cast<const uint4*>(p + 16 * k);
-      q[2 * k] = make_uint2(v.x, v.y);
-      q[2 * k + 1] = make_uint2(v.z, v.w);
-    }
-  }
-  __device__ __forceinline__ void load_quads(const uint8_t* p, int m0, int m1) {
-#pragma unroll
-    for (int m = 0; m < MT; ++m)
-      if (m >= m0 && m < m1) q[m] = *reinterpret_cast<const uint2*>(p + 8 * m);
-  }
-  // the same loads through a buffer resource: per-lane offset voff, uniform
-  // offset soff (bytes)
-  __device__ __forceinline__ void bload(__amdgpu_buffer_rsrc_t r, uint32_t voff, int soff) {
-#pragma unroll
-    for (int k = 0; k < MT / 2; ++k) {
-      const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(r, voff + 16 * k, soff, 0);
-      q[2 * k] = make_uint2(v.x, v.y);
-      q[2 * k + 1] = make_uint2(v.z, v.w);
-    }
-  }
-  __device__ __forceinline__ void bload_quads(__amdgpu_buffer_rsrc_t r, uint32_t voff, int soff, int m0, int m1) {
-#pragma unroll
-    for (int m = 0; m < MT; ++m)
-      if (m >= m0 && m < m1) {
-        const u32x2 v = __builtin_amdgcn_raw_buffer_load_b64(r, voff + 8 * m, soff, 0);
-        q[m] = make_uint2(v.x, v.y);
-      }
-  }
-  __device__ __forceinline__ void store_quads(uint8_t* p, int m0, int m1) const {
-#pragma unroll
-    for (int m = 0; m < MT; ++m)
-      if (m >= m0 && m < m1) *reinterpret_cast<uint2*>(p + 8 * m) = q[m];
-  }
-  __device__ __forceinline__ void store(uint8_t* p) const {
-#pragma unroll
-    for (int k = 0; k < MT / 2; ++k)
-      *reinterpret_cast<uint4*>(p + 16 * k) = make_uint4(q[2 * k].x, q[2 * k].y, q[2 * k + 1].x, q[2 * k + 1].y);
-  }
-  __device__ __forceinline__ void bstore_quads(__amdgpu_buffer_rsrc_t r, uint32_t voff, int soff, int m0,
-                                               int m1) const {
-#pragma unroll
-    for (int m = 0; m < MT; ++m)
-      if (m >= m0 && m < m1) __builtin_amdgcn_raw_buffer_store_b64(u32x2{q[m].x, q[m].y}, r, voff + 8 * m, soff, 0);
-  }
-  __device__ __forceinline__ void bstore(__amdgpu_buffer_rsrc_t r, uint32_t voff, int soff) const {
-#pragma unroll
-    for (int k = 0; k < MT / 2; ++k)
-      __builtin_amdgcn_raw_buffer_store_b128(u32x4{q[2 * k].x, q[2 * k].y, q[2 * k + 1].x, q[2 * k + 1].y}, r,
-                                             voff + 16 * k, soff, 0);
-  }
-  __device__ __forceinline__ void set(int m, f32x4 v) {
-    typename Prec<PREC>::quad h = to_quad<PREC>(v);
-    q[m] = *reinterpret_cast<uint2*>(&h);
-  }
-  __device__ __forceinline__ f32x4 get(int m) const {
-    return from_quad<PREC>(*reinterpret_cast<const typename Prec<PREC>::quad*>(&q[m]));
-  }
-  template <int KS>
-  __device__ __forceinline__ void frags(typename Prec<PREC>::frag (&b)[KS]) const {
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks) {
-      uint4 v = make_uint4(q[2 * ks].x, q[2 * ks].y, q[2 * ks + 1].x, q[2 * ks + 1].y);
-      b[ks] = *reinterpret_cast<typename Prec<PREC>::frag*>(&v);
-    }
-  }
-};
-
-template <int C>
-struct LaneData<FK_PREC_FP32, C> {
-  static constexpr int MT = C / 16;
-  static constexpr int LB = MT * 16;
-  f32x4 q[MT];
-  __device__ __forceinline__ void load(const uint8_t* p) {
-#pragma unroll
-    for (int m = 0; m < MT; ++m) q[m] = *reinterpret_cast<const f32x4*>(p + 16 * m);
-  }
-  __device__ __forceinline__ void load_quads(const uint8_t* p, int m0, int m1) {
-#pragma unroll
-    for (int m = 0; m < MT; ++m)
-      if (m >= m0 && m < m1) q[m] = *reinterpret_cast<const f32x4*>(p + 16 * m);
-  }
-  __device__ __forceinline__ void store_quads(uint8_t* p, int m0, int m1) const {
-#pragma unroll
-    for (int m = 0; m < MT; ++m)
-      if (m >= m0 && m < m1) *reinterpret_cast<f32x4*>(p + 16 * m) = q[m];
-  }
-  __device__ __forceinline__ void store(uint8_t* p) const { store_quads(p, 0, MT); }
-  __device__ __forceinline__ void set(int m, f32x4 v) { q[m] = v; }
-  __device__ __forceinline__ f32x4 get(int m) const { return q[m]; }
-  template <int KS>
-  __device__ __forceinline__ void frags(float (&b)[KS]) const {
-#pragma unroll
-    for (int t = 0; t < KS; ++t) b[t] = q[t >> 2][t & 3];
-  }
-};
 
 // Per-lane activation loads of one horizontal-stack block step of the fast
 // sampler (from the per-tile cache in HBM): the two earlier horizontal-stack
@@ -157,25 +50,9 @@ struct VLoads {
   LaneData<PREC, C> vr;
 };
 
-struct SampArgs {
-  const void* w;
-  const float* aux;
-  int H, W, HW, nb;
-  int64_t batch;
-  const double* uniforms;
-  int8_t* out;
-  float* cond;
-  uint8_t* cache;
-  int64_t tile_bytes;
-};
-
 // WR: the whole-row vertical pass (16-bit 32-channel nets, rows of at most
 // VROW_MAX pixels), with its rows in dynamic LDS (fast_vrow_lds bytes).
 constexpr int VROW_MAX = 10;
-template <int PREC, int C>
-constexpr int fast_lb() {
-  return PREC == FK_PREC_FP32 ? (C / 16) * 16 : (C / 16) * 8;
-}
 inline int fast_vrow_lds(int W, int lb) { return (6 * W + 1) * 64 * lb + 3 * W * 16 * 4; }
 
 // Whether a block step's operands are all requested ahead of its MFMAs (the
@@ -187,11 +64,6 @@ struct FastBatch {
       (C / 16) * (C / Prec<PREC>::KW) * (int)(sizeof(typename Prec<PREC>::frag) / 4) <= 8;
   static constexpr int unr = value ? 9 : 1;
 };
-
-// Four consecutive biases of one lane group (16-byte aligned: every bias
-// offset of the aux buffer is a multiple of 4 floats, and channels 16 m + 4 g
-// .. + 3 stay inside the C or C/2 biases of the M-tiles that read them).
-__device__ __forceinline__ f32x4 ldq4(const float* p) { return *reinterpret_cast<const f32x4*>(p); }
 
 template <int PREC, int C, int ACT, bool WR>
 __global__ __launch_bounds__(64) void fast_sample_kernel(SampArgs a) {
@@ -1159,6 +1031,7 @@ static bool fast_whole_row(int W, int channels, int precision) {
 // and, for the whole-row kernel, one row of concatenation partial sums per
 // block (FP32, MT quads per lane, VROW_MAX columns).
 int64_t fast_tile_bytes(int H, int W, int nb, int channels, int precision) {
+  if (fast_mw_supported(H, W, nb, channels, precision)) return fast_mw_tile_bytes(H, W, nb, channels, precision);
   const int esz = precision == FK_PREC_FP32 ? 4 : 2;
   const int64_t pb = 16LL * channels * esz;
   const int64_t HW = (int64_t)H * W;
@@ -1234,6 +1107,7 @@ int fk_fast_sample(const void* wpacked, const float* aux, int32_t precision, int
   const int64_t tiles = (batch + 15) / 16;
   FK_REQUIRE(tiles <= 0x7fffffff, "fk_fast_sample: batch too large");
   hipStream_t s = (hipStream_t)stream;
+  if (fast_mw_supported(H, W, a.nb, CP, precision)) return launch_fast_mw(a, CP, precision, activation, tiles, s);
   if (precision == FK_PREC_BF16) {
     if (CP == 32) return launch_fast<FK_PREC_BF16, 32>(a, activation, tiles, s);
     return launch_fast<FK_PREC_BF16, 64>(a, activation, tiles, s);

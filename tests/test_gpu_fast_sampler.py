@@ -68,3 +68,24 @@ def test_fast_sampler_chunks(rng):
     a = next(fk.FastAutoregressiveSampler(m, 50, uniforms=u))
     b = next(fk.FastAutoregressiveSampler(m, 50, mini_batch_size=16, uniforms=u))
     assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize('shape,depth,C,act,prec,B', [((5, 6), 4, 32, 'elu', 'fp16', 17),
+                                                      ((3, 1), 5, 32, 'relu', 'bf16', 16),
+                                                      ((1, 9), 5, 24, 'elu', 'fp16', 5),
+                                                      ((4, 13), 10, 32, 'relu', 'fp16', 40),
+                                                      ((3, 40), 9, 20, 'elu', 'bf16', 20),
+                                                      ((6, 5), 12, 64, 'elu', 'bf16', 33),
+                                                      ((4, 26), 6, 48, 'relu', 'fp16', 18),
+                                                      ((3, 39), 4, 64, 'relu', 'bf16', 16),
+                                                      ((7, 7), 20, 32, 'elu', 'bf16', 20),
+                                                      ((4, 6), 10, 32, 'relu', 'fp32', 19),
+                                                      ((3, 14), 5, 48, 'elu', 'fp32', 17),
+                                                      ((3, 21), 9, 64, 'relu', 'fp32', 16)])
+def test_workgroup_per_tile_equals_plain(rng, shape, depth, C, act, prec, B):
+    """The workgroup-per-tile kernel: one to seven steps per super-tick (and a
+    last super-tick that is not full), rows of one pixel, rows that the waves
+    take in several groups, the widest rows the LDS holds, each kernel width
+    and precision.  Draws and conditionals are those of the plain sampler, bit
+    for bit."""
+    test_fast_equals_plain_given_uniforms(rng, shape, depth, C, act, prec, B)
