@@ -11,85 +11,13 @@
 // into O_re and O_im (batch, P) in the canonical flat parameter order.
 // Derivatives of the activations are taken from the stored outputs
 // (relu' = [y > 0], elu' = y > 0 ? 1 : y + 1).
-#include "fk_common.h"
-#include "convar_layout.h"
+//
+// 32 and 64 channels take convar_grad.hip (grad_plan); this file's MFMA kernels
+// the larger multiples of 32, and operands that are not aligned to 16 bytes;
+// the scalar kernel the other widths.
+#include "convar_bwd.h"
 
 namespace fk {
-
-template <int ACT>
-__device__ __forceinline__ float bact(float x) {
-  if constexpr (ACT == FK_ACT_RELU) return fmaxf(x, 0.0f);
-  else return x > 0.0f ? x : expm1f(x);
-}
-template <int ACT>
-__device__ __forceinline__ float bdact(float y) {  // derivative from the output
-  if constexpr (ACT == FK_ACT_RELU) return y > 0.0f ? 1.0f : 0.0f;
-  else return y > 0.0f ? 1.0f : y + 1.0f;
-}
-
-struct BwdArgs {
-  const float* params;  // flat parameters (effective kernels), P floats
-  int H, W, HW, C, nb;
-  int64_t batch;
-  const int8_t* spins;  // (batch, HW)
-  float* work;          // per-workgroup activation store
-  int64_t work_floats;  // floats per workgroup
-  float* o_re;          // (batch, P)
-  float* o_im;
-  float* logpsi;        // (batch, 2) or null
-  int64_t P;
-  int64_t ld;           // row stride of o_re / o_im (>= P)
-  const float* cot;     // GRAD_VJP: (batch, 2) cotangents of (Re, Im) log psi
-  float* partial;       // GRAD_VJP: (gridDim.x, P) per-workgroup partial gradients
-  const float* tangent; // JVP: direction, P floats
-  float* jvp;           // JVP: (batch, 2) output
-  const float* kt;      // the conv kernels transposed (transpose_kernels_kernel), P floats
-  const float* tkt;     // JVP: the tangent's conv kernels transposed
-  int stage;            // LDS row stride (floats) of the two staging tiles, 0: no staging
-};
-
-// Offsets of layer parameters in the flat vector.
-struct ParamOffsets {
-  int64_t kv, bv, kh, bh, kx, bx, ky, by, kc, bc;
-};
-__device__ __forceinline__ ParamOffsets param_offsets(int blk, int C) {
-  // block 0 has cin = 1; blocks >= 1 have cin = C
-  const int64_t blk0 = 9LL * C + C + 3LL * C + C + (int64_t)C * (C / 2) * 2 + C + 9LL * C * C + C;
-  const int64_t blkn = 9LL * C * C + C + 3LL * C * C + C + (int64_t)C * (C / 2) * 2 + C + 9LL * C * C + C;
-  const int64_t base = blk == 0 ? 0 : blk0 + (int64_t)(blk - 1) * blkn;
-  const int cin = blk == 0 ? 1 : C;
-  ParamOffsets o;
-  o.kv = base;
-  o.bv = o.kv + 9LL * cin * C;
-  o.kh = o.bv + C;
-  o.bh = o.kh + 3LL * cin * C;
-  o.kx = o.bh + C;
-  o.bx = o.kx + (int64_t)C * (C / 2);
-  o.ky = o.bx + C / 2;
-  o.by = o.ky + (int64_t)C * (C / 2);
-  o.kc = o.by + C / 2;
-  o.bc = o.kc + 9LL * C * C;
-  return o;
-}
-__device__ __forceinline__ int64_t head_offset(int nb, int C) {
-  const ParamOffsets o = param_offsets(nb - 1, C);
-  return o.bc + C;
-}
-
-// Tap offsets: vertical kxk rows -2..0 cols -1..1; horizontal 1xk cols -2..0;
-// h3 kxk rows -2..0 cols -2..0.
-__device__ __forceinline__ void tap_rc(int kind, int t, int& dr, int& dc) {
-  if (kind == 0) {
-    dr = t / 3 - 2;
-    dc = t % 3 - 1;
-  } else if (kind == 1) {
-    dr = 0;
-    dc = t - 2;
-  } else {
-    dr = t / 3 - 2;
-    dc = t % 3 - 2;
-  }
-}
 
 // out[p][co] = b[co] + sum_{tap,ci} K[tap][ci][co] * in[p + off][ci]
 // (cin channels; in/out are [HW][cs] with channel strides cs_in/cs_out).
@@ -170,15 +98,6 @@ __device__ void conv_bwd_weight(float* dK, float* db, const float* in, int cs_in
   }
 }
 
-// Per-sample workspace layout (floats): spins HW, then per block
-// VA (act(v')), XA (act(hx)), CAT (x2|y2), VO (vertical output), HO
-// (horizontal output), each HW*C.
-// (the spins region is padded to 4 floats so that every tensor is 16-byte
-// aligned)
-__device__ __forceinline__ float* ws_tensor(float* ws, int HW, int C, int blk, int which) {
-  return ws + ((HW + 3) & ~3) + ((int64_t)blk * 5 + which) * HW * C;
-}
-enum { T_VA = 0, T_XA = 1, T_CAT = 2, T_VO = 3, T_HO = 4 };
 
 template <int ACT>
 __global__ __launch_bounds__(256) void convar_grad_kernel(BwdArgs a) {
@@ -429,14 +348,6 @@ __global__ __launch_bounds__(256) void convar_grad_kernel(BwdArgs a) {
 // MFMA 16x16x4 lane roles: A[i][k] in lane i + 16k, B[k][j] in lane j + 16k,
 // D[i][j] in lane j + 16*(i/4), register i%4.
 
-// source-table rows: vertical taps 0-8, horizontal 9-11, h3 12-20, x1x1 21,
-// x1x1 behind the RightShift (final block) 22, y1x1 behind the DownShift 23
-constexpr int GT_V = 0, GT_H = 9, GT_C = 12, GT_X = 21, GT_XF = 22, GT_Y = 23, GT_N = 24;
-
-__device__ __forceinline__ f32x4 mfma4(float a, float b, f32x4 c) {
-  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-}
-
 // Each wave walks 2x2 blocks of 16x16 D tiles; the K loop is (outer, inner)
 // so that tap and channel-quad indices need no division.
 template <class FA, class FB, class FS>
@@ -527,20 +438,6 @@ __global__ void transpose_kernels_kernel(const float* __restrict__ prm, float* _
     const int ci = rem / cout, co = rem - (rem / cout) * cout;
     kt[off + ((int64_t)t * cout + co) * cin + ci] = prm[off + e];
   }
-}
-
-// Elementwise passes over HW x C tensors (C a multiple of 4) in 16-byte
-// vectors: element i of a tensor as a quad, the activation and its
-// derivative per component.
-__device__ __forceinline__ f32x4 L4(const float* p, int i) { return *reinterpret_cast<const f32x4*>(p + 4 * i); }
-__device__ __forceinline__ f32x4& S4(float* p, int i) { return *reinterpret_cast<f32x4*>(p + 4 * i); }
-template <int ACT>
-__device__ __forceinline__ f32x4 bact4(f32x4 x) {
-  return f32x4{bact<ACT>(x[0]), bact<ACT>(x[1]), bact<ACT>(x[2]), bact<ACT>(x[3])};
-}
-template <int ACT>
-__device__ __forceinline__ f32x4 bdact4(f32x4 y) {
-  return f32x4{bdact<ACT>(y[0]), bdact<ACT>(y[1]), bdact<ACT>(y[2]), bdact<ACT>(y[3])};
 }
 
 // Copies n channels (from channel off, row stride cs) of an HW-pixel tensor
@@ -689,12 +586,6 @@ __device__ void mconv_bwd_weight(float* dK, float* db, const float* in, int cs_i
       else db[co] = acc;
     }
   }
-}
-
-// Per-sample workspace of the MFMA kernel: the scalar kernel's layout plus six
-// gradient tensors (dV, dH, dVr, dHr, t0, t1) of HW*C floats.
-__device__ __forceinline__ float* ws_grad(float* ws, int HW, int C, int nb, int which) {
-  return ws + ((HW + 3) & ~3) + ((int64_t)nb * 5 + which) * HW * C;
 }
 
 // Source tables (and their inverses) of every tap / shift of the lattice.
@@ -884,15 +775,6 @@ __device__ __forceinline__ void mfma_forward(const float* prm, const float* tan,
   }
 }
 
-// Head logits z[k] (k = 0, 1: Re for spin +1 / -1; 2, 3: Im) of pixel p.
-__device__ __forceinline__ void head_logits(const float* prm, int64_t ho, const float* HF, int C, int p, float z[4]) {
-  for (int k = 0; k < 4; ++k) {
-    float acc = prm[ho + 4 * C + k];
-    for (int ci = 0; ci < C; ++ci) acc += prm[ho + ci * 4 + k] * HF[p * C + ci];
-    z[k] = acc;
-  }
-}
-
 // Backward of one sample from the head cotangent dz (HW x 4): d/d theta into
 // O (overwritten, or added to when accumulate).
 template <int ACT, bool ACC, bool STG>
@@ -1009,7 +891,6 @@ __device__ __forceinline__ void mfma_backward(const float* prm, float* ws, const
   __syncthreads();
 }
 
-enum { GRAD_O = 0, GRAD_VJP = 1 };
 
 // MODE GRAD_O: one workgroup per sample, O_re / O_im rows from two backward
 // passes (cotangents of Re and Im log psi).  MODE GRAD_VJP: a persistent grid,
@@ -1163,6 +1044,7 @@ __global__ void reduce_partials_kernel(const float* __restrict__ part, int64_t n
   const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (q >= P) return;
   double acc = 0.0;
+#pragma unroll 16
   for (int64_t g = 0; g < nparts; ++g) acc += (double)part[g * P + q];
   out[q] = (float)(scale * acc);
 }
@@ -1198,10 +1080,10 @@ int stage_stride(int HW, int C) {
   const size_t b = grad_lds_bytes(HW) + (size_t)2 * HW * SC * sizeof(float);
   return (C % 4 == 0 && b <= GRAD_LDS_PER_WG) ? SC : 0;
 }
-// Workgroups per CU of the batched VJP: four with staging tiles (128 VGPRs,
-// 24.1 ms per 2048 samples at 10x10/C32 against 27.9 at three), three
-// without (the unstaged 20x20/C64 implicit products of 16384 samples took
-// 430 us per sample at three, 472 at four).
+// Workgroups per CU of the batched VJP: four with staging tiles (128 VGPRs),
+// three without.  (The line was drawn with this kernel at 10x10 C 32, 2048
+// samples: 24.1 ms at four, 27.9 at three; and unstaged at 20x20 C 64, 16384
+// samples: 430 us a sample at three, 472 at four.)
 int vjp_per_cu(int HW, int C) { return stage_stride(HW, C) ? 4 : 3; }
 size_t grad_lds_total(int HW, int stage) {
   return grad_lds_bytes(HW) + (stage ? (size_t)2 * HW * stage * sizeof(float) : 0);
@@ -1244,7 +1126,7 @@ extern "C" {
 int64_t fk_convar_grad_workspace_bytes(int32_t H, int32_t W, int32_t depth, int32_t channels, int64_t batch) {
   if (H < 1 || W < 1 || depth < 1 || channels < 2 || (channels % 2) || batch < 0) return -1;
   const int nb = num_causal_blocks(depth);
-  return (kt_floats(channels, nb) + batch * grad_work_floats(H * W, channels, nb)) * (int64_t)sizeof(float);
+  return (2 * kt_floats(channels, nb) + batch * grad_work_floats(H * W, channels, nb)) * (int64_t)sizeof(float);
 }
 
 int fk_convar_grad(const float* params, int32_t H, int32_t W, int32_t depth, int32_t channels, int32_t activation,
@@ -1265,7 +1147,8 @@ int fk_convar_grad(const float* params, int32_t H, int32_t W, int32_t depth, int
   a.batch = batch;
   a.spins = spins;
   a.kt = reinterpret_cast<float*>(workspace);
-  a.work = reinterpret_cast<float*>(workspace) + kt_floats(channels, a.nb);
+  a.kb = a.kt + kt_floats(channels, a.nb);
+  a.work = reinterpret_cast<float*>(workspace) + 2 * kt_floats(channels, a.nb);
   a.work_floats = grad_work_floats(a.HW, channels, a.nb);
   a.o_re = o_re;
   a.o_im = o_im;
@@ -1279,6 +1162,8 @@ int fk_convar_grad(const float* params, int32_t H, int32_t W, int32_t depth, int
     a.stage = stage_stride(a.HW, channels);
     const size_t lds = grad_lds_total(a.HW, a.stage);
     FK_REQUIRE(lds <= 160 * 1024 && a.HW <= 32767, "fk_convar_grad: lattice too large");
+    const GradPlan plan = grad_plan(a, GRAD_O);
+    if (plan.threads) return launch_grad_plan(plan, a, activation, GRAD_O, s);
     const int rc = launch_transpose(params, const_cast<float*>(a.kt), channels, a.nb, s);
     if (rc != FK_OK) return rc;
     return activation == FK_ACT_ELU
@@ -1306,7 +1191,7 @@ int64_t fk_convar_vjp_workspace_bytes(int32_t H, int32_t W, int32_t depth, int32
   if (H < 1 || W < 1 || depth < 1 || channels < 32 || (channels % 32) || batch < 0) return -1;
   const int nb = num_causal_blocks(depth);
   const int64_t g = implicit_grid(batch, vjp_per_cu(H * W, channels));
-  return (kt_floats(channels, nb) + g * (grad_work_floats(H * W, channels, nb) + flat_param_count(channels, nb))) *
+  return (2 * kt_floats(channels, nb) + g * (grad_work_floats(H * W, channels, nb) + flat_param_count(channels, nb))) *
          (int64_t)sizeof(float);
 }
 
@@ -1328,21 +1213,28 @@ int fk_convar_vjp(const float* params, int32_t H, int32_t W, int32_t depth, int3
   a.batch = batch;
   a.spins = spins;
   a.kt = reinterpret_cast<float*>(workspace);
-  a.work = reinterpret_cast<float*>(workspace) + kt_floats(channels, a.nb);
+  a.kb = a.kt + kt_floats(channels, a.nb);
+  a.work = reinterpret_cast<float*>(workspace) + 2 * kt_floats(channels, a.nb);
   a.work_floats = grad_work_floats(a.HW, channels, a.nb);
   a.logpsi = logpsi;
   a.P = flat_param_count(channels, a.nb);
   a.cot = cot;
-  const int64_t g = implicit_grid(batch, vjp_per_cu(H * W, channels));
+  const GradPlan plan = grad_plan(a, GRAD_VJP);
+  const int64_t g = plan.threads ? plan.grid : implicit_grid(batch, vjp_per_cu(H * W, channels));
   a.partial = a.work + g * a.work_floats;
   a.stage = stage_stride(a.HW, channels);
   const size_t lds = grad_lds_total(a.HW, a.stage);
   FK_REQUIRE(lds <= 160 * 1024 && a.HW <= 32767, "fk_convar_vjp: lattice too large");
   hipStream_t s = (hipStream_t)stream;
-  int rc = launch_transpose(params, const_cast<float*>(a.kt), channels, a.nb, s);
-  if (rc != FK_OK) return rc;
-  rc = activation == FK_ACT_ELU ? launch_grad<FK_ACT_ELU, GRAD_VJP>(g, lds, s, a)
-                                : launch_grad<FK_ACT_RELU, GRAD_VJP>(g, lds, s, a);
+  int rc;
+  if (plan.threads) {
+    rc = launch_grad_plan(plan, a, activation, GRAD_VJP, s);
+  } else {
+    rc = launch_transpose(params, const_cast<float*>(a.kt), channels, a.nb, s);
+    if (rc != FK_OK) return rc;
+    rc = activation == FK_ACT_ELU ? launch_grad<FK_ACT_ELU, GRAD_VJP>(g, lds, s, a)
+                                  : launch_grad<FK_ACT_RELU, GRAD_VJP>(g, lds, s, a);
+  }
   if (rc != FK_OK) return rc;
   hipLaunchKernelGGL(reduce_partials_kernel, dim3(div_up(a.P, 256)), dim3(256), 0, s, a.partial, g, a.P, scale,
                      grad);
@@ -1387,6 +1279,8 @@ int fk_convar_jvp(const float* params, const float* tangent, int32_t H, int32_t 
   FK_REQUIRE(lds <= 160 * 1024 && a.HW <= 32767, "fk_convar_jvp: lattice too large");
   const int64_t g = implicit_grid(batch, JVP_PER_CU);
   hipStream_t s = (hipStream_t)stream;
+  const GradPlan plan = grad_plan(a, GRAD_JVP);
+  if (plan.threads) return launch_grad_plan(plan, a, activation, GRAD_JVP, s);
   int rc = launch_transpose(params, const_cast<float*>(a.kt), channels, a.nb, s);
   if (rc == FK_OK) rc = launch_transpose(tangent, const_cast<float*>(a.tkt), channels, a.nb, s);
   if (rc != FK_OK) return rc;

@@ -198,6 +198,61 @@ def test_mfma_per_sample_gradients_vs_autograd(rng, shape, depth, C, act):
     assert np.abs(lp[:, 0].cpu().numpy() - ref.real).max() < 1e-4 * (np.abs(ref.real).max() + 1)
 
 
+# One pixel; less than a tile and a tile more or less; one, two and four
+# workgroups per CU and more samples than workgroups; tensors in LDS and in the
+# workspace; the widest lattice in LDS of each width; 96 channels.
+@pytest.mark.parametrize('shape,depth,C,act,B', [
+    ((1, 1), 2, 32, 'elu', 3), ((3, 5), 3, 32, 'relu', 5), ((4, 4), 3, 32, 'elu', 1030), ((1, 17), 2, 64, 'elu', 4),
+    ((5, 7), 2, 64, 'elu', 300), ((7, 7), 3, 32, 'relu', 300), ((9, 11), 4, 32, 'elu', 2), ((12, 12), 3, 32, 'elu', 3),
+    ((13, 14), 2, 32, 'elu', 300), ((8, 11), 2, 64, 'elu', 3), ((11, 12), 2, 64, 'elu', 260), ((4, 5), 3, 96, 'elu', 5)])
+def test_gradient_kernels_over_tiles_and_grids(rng, shape, depth, C, act, B):
+    """Per-sample O of three samples against float64 autograd; VJP and JVP
+    of the whole batch against products with O; rows of an odd stride and
+    parameters off 16 bytes.  FP32 sums of up to 9 C terms through 2 depth
+    convolutions: the bounds of the tests above."""
+    gpu_banner(f'gradient kernels shape={shape} depth={depth} C={C} {act} B={B}')
+    import flowket_amd as fk
+    from flowket_amd import _lib
+    m = fk.ConvNetAutoregressive2D(shape, depth=depth, num_of_channels=C, activation=act,
+                                   weights_normalization=False, precision='fp32', seed=6)
+    g = torch.Generator().manual_seed(7)
+    p = m.params.cpu() * (1.0 + 0.3 * torch.randn(m.n_params, generator=g))
+    m.set_params(p + 0.05 * torch.randn(m.n_params, generator=g) * (p == 0))
+    s = rng.choice([-1, 1], size=(B,) + shape).astype(np.int8)
+    o_re, o_im, lp = m.per_sample_gradients(s)
+    O = o_re.double().cpu().numpy() + 1j * o_im.double().cpu().numpy()
+    pick = sorted({0, B // 2, B - 1})
+    flat = m.params.double().cpu().clone().requires_grad_(True)
+    re, im = _torch_log_psi(flat, m.shapes, s[pick], depth, act)
+    for k, b in enumerate(pick):
+        j = torch.autograd.grad(re[k], flat, retain_graph=True)[0].numpy() + \
+            1j * torch.autograd.grad(im[k], flat, retain_graph=True)[0].numpy()
+        assert np.abs(O[b] - j).max() / np.abs(j).max() < 1e-4
+        assert abs(lp[b, 0].item() - re[k].item()) < 1e-4 * (abs(re[k].item()) + 1)
+    u = rng.normal(size=(B, 2))
+    got = m.vjp(s, torch.as_tensor(u, dtype=torch.float32), 0.5).double().cpu().numpy()
+    ref = 0.5 * (O.real.T @ u[:, 0] + O.imag.T @ u[:, 1])
+    assert np.abs(got - ref).max() < 2e-5 * np.abs(ref).max()
+    t = rng.normal(size=m.n_params)
+    w = m.jvp(s, torch.as_tensor(t, dtype=torch.float32)).double().cpu().numpy()
+    ref_w = O @ t
+    assert np.abs(w - np.stack([ref_w.real, ref_w.imag], 1)).max() < 2e-5 * np.abs(ref_w).max()
+
+    P, ld = m.n_params, m.n_params + 3
+    spins = torch.as_tensor(s.reshape(B, -1)).to(m.device)
+    ws = torch.empty(_lib.load().fk_convar_grad_workspace_bytes(*shape, depth, C, B), dtype=torch.uint8, device=m.device)
+    off = torch.empty(P + 1, device=m.device)[1:]
+    off.copy_(m.params)
+    for params in (m.params, off):
+        rows = torch.zeros(2, B * ld + 1, device=m.device)
+        _lib.call('fk_convar_grad', _lib.ptr(params), *shape, depth, C, {'relu': 0, 'elu': 1}[act], _lib.ptr(spins), B,
+                  _lib.ptr(ws), rows[0, 1:].data_ptr(), rows[1, 1:].data_ptr(), ld, None, _lib.stream_ptr())
+        r = rows[:, 1:].reshape(2, B, ld)
+        assert not r[:, :, P:].any()
+        for got, want in zip(r, (o_re, o_im)):
+            assert (got[:, :P] - want).abs().max().item() < 1e-5 * np.abs(O).max()
+
+
 @pytest.mark.parametrize('B,P', [(37, 1000), (37, 1001), (5, 4)])
 def test_sr_products_c_abi(rng, B, P):
     """fk_o_times_v / fk_oh_times_u on random O against dense float64 algebra,
