@@ -64,11 +64,19 @@ static int current_schedule(int H, int W, int depth, int C, int act, int prec) {
   return it == g_sched.end() ? 0 : it->second;
 }
 
-// Largest tile of configurations whose activation lattices fit in the 160 KB
-// LDS with at most 4 (8 waves) or 8 (4 waves) 16-pixel tiles per wave.
+// Tile of configurations: at most what fits the 160 KB LDS with at most 4 (8
+// waves) or 8 (4 waves) 16-pixel tiles per wave.  The launch then needs
+// `rounds` groups on each of its workgroups, and the tile is the smallest that
+// needs no more: a group of fewer configurations is faster, and few
+// configurations are spread over the chip.  (m is the number of configurations
+// or, for device counts, their bound; the 16-bit kernels repeat the rule on the
+// count itself.)  Against the largest tile always, us: 16 of 4x4 C 16 FP32 70 ->
+// 60, 600 of 5x7 C 32 fp16 49 -> 29, 10x10 C 32 depth 20 fp16 64 217 -> 134, 512
+// 217 -> 155, 2048 420 -> 390, 4096 830 -> 770 (four rounds of four, not of five).
 // HWL: LDS pixels per configuration, HWC: computed pixels per configuration
 // (they differ for row-reuse launches, whose halo rows are not computed).
-static int plan_forward(int HWL, int HWC, int C, int prec, int NW, int64_t m, FwdPlan* plan, bool hg = false) {
+static int plan_forward(int HWL, int HWC, int C, int prec, int NW, int64_t m, FwdPlan* plan, bool hg = false,
+                        bool exact = true) {
   const int pixb = C * (prec == FK_PREC_FP32 ? 4 : 2);
   const size_t cap = FWD_DYN_LDS;
   const int maxt_cap = (NW == 4) ? 8 : 4;
@@ -82,12 +90,17 @@ static int plan_forward(int HWL, int HWC, int C, int prec, int NW, int64_t m, Fw
     if ((int64_t)T >= m) break;
   }
   if (best == 0) return FK_ERR_UNSUPPORTED;
+  plan->lds = fwd_lds_bytes(best * HWL, pixb, hg, best);
+  plan->slots = (int64_t)device_cu_count() * fwd_per_cu(*plan);
+  if (exact) {
+    best = fwd_tile(best, m, plan->slots);
+    plan->lds = fwd_lds_bytes(best * HWL, pixb, hg, best);
+  }
   plan->T = best;
   plan->npix = ((best * HWC + 15) / 16) * 16;
-  plan->lds = fwd_lds_bytes(best * HWL, pixb, hg, best);
   plan->nwave = NW;
   const int per_wave = (plan->npix / 16 + NW - 1) / NW;
-  plan->maxt = per_wave <= 2 ? 2 : (per_wave <= 4 ? 4 : 8);
+  plan->maxt = per_wave <= 1 ? 1 : per_wave <= 2 ? 2 : (per_wave <= 4 ? 4 : 8);
   return FK_OK;
 }
 
@@ -233,8 +246,7 @@ static int64_t forward_workspace_bytes(int H, int W, int depth, int CP, int act,
     const int hr = r0 == 0 ? H : H - r0 + 2, hc = r0 == 0 ? H : H - r0;
     FwdPlan q;
     if (plan_forward(hr * W, hc * W, CP, prec, hg_waves(table[si]), 1 << 30, &q, true) != FK_OK) return -1;
-    const int per_cu = fwd_per_cu(q);
-    const int64_t b = (int64_t)device_cu_count() * per_cu * 2 * (int64_t)(q.T * hr * W + ZERO_PIX) * pixb;
+    const int64_t b = q.slots * 2 * (int64_t)(q.T * hr * W + ZERO_PIX) * pixb;
     if (b > need) need = b;
   }
   return need;
@@ -301,8 +313,9 @@ static int convar_forward(const void* wpacked, const float* aux, int32_t precisi
   a.m_range = rr.m_range;
   const int HWL = a.HR * W, HWC = a.HC * W;
   hipStream_t s = (hipStream_t)stream;
+  const bool exact = !m_dev && !rr.m_range;
   FwdPlan pl;
-  if (plan_forward(HWL, HWC, CP, precision, sc.nwave, m_count, &pl) != FK_OK) {
+  if (plan_forward(HWL, HWC, CP, precision, sc.nwave, m_count, &pl, false, exact) != FK_OK) {
     // horizontal stack in global scratch
     FwdPlan hp;
     const int64_t need = forward_workspace_bytes(H, W, depth, CP, activation, precision, &hp);
@@ -316,7 +329,7 @@ static int convar_forward(const void* wpacked, const float* aux, int32_t precisi
                 "(fk_convar_forward_workspace_bytes, fk_convar_forward_ws)", H, W, channels, (long long)need);
       return FK_ERR_ARG;
     }
-    if (plan_forward(HWL, HWC, CP, precision, hg_waves(sc), m_count, &pl, true) != FK_OK) return FK_ERR_UNSUPPORTED;
+    if (plan_forward(HWL, HWC, CP, precision, hg_waves(sc), m_count, &pl, true, exact) != FK_OK) return FK_ERR_UNSUPPORTED;
     if (fwd_grid(a, pl) * 2 * (int64_t)(pl.T * HWL + ZERO_PIX) * (CP * (precision == FK_PREC_FP32 ? 4 : 2)) >
         workspace_bytes) {
       set_error("ConvNetAutoregressive2D kernels: workspace too small for this launch");

@@ -148,6 +148,15 @@ struct Lds {
   }
 };
 
+// Configurations per group, at most best, for m of them on slots workgroups:
+// the smallest that needs no more rounds.
+__host__ __device__ __forceinline__ int fwd_tile(int best, int64_t m, int64_t slots) {
+  if (m <= 0 || m > 0x7fffffff) return best;
+  const uint32_t M = (uint32_t)m, S = (uint32_t)slots;
+  const uint32_t rounds = (M + best * S - 1) / (best * S);
+  return (int)((M + rounds * S - 1) / (rounds * S));
+}
+
 struct FwdArgs {
   const void* w;
   const float* aux;
@@ -445,15 +454,28 @@ __global__ __launch_bounds__(64 * NWAVE) void convar_fwd_kernel(FwdArgs a) {
   const ConvarLayout lay(C, PREC);
 
   extern __shared__ __align__(16) uint8_t lds[];
-  // npix: pixels covered by the 16-pixel tiles; NPX = T*HW real pixels.
+  auto count = [&](int64_t& m0) {
+    int64_t M = a.m_dev ? *a.m_dev : a.m_count;
+    m0 = 0;
+    if (a.m_range) {
+      m0 = a.m_range[0];
+      M = a.m_range[1] - m0;
+    }
+    return M > a.m_count ? a.m_count : M;
+  };
+  int64_t m0, M = 0;
+  // (not in FP32, where 512 10x10 C 32 depth 20 configurations took 1.11 ms with
+  // a.T and 1.14 to 1.16 with a tile computed here)
+  if constexpr (PREC != FK_PREC_FP32) M = count(m0);
+  const int T = PREC == FK_PREC_FP32 ? a.T : __builtin_amdgcn_readfirstlane(fwd_tile(a.T, M, gridDim.x));
+  // NPX = T*HW real pixels, covered by 16-pixel tiles.
   // Each buffer holds the NPX pixels plus ZERO_PIX all-zero pixels that padding
   // taps and the tile lanes past NPX read: a lane whose tap target q falls
   // outside reads zero pixel NPX + ((q - NPX) & 7), which has the bank
   // placement q itself would have, so border tiles stay conflict-free.
-  const int npix = a.npix;
   // per configuration: HWL pixels in LDS (halo rows included), HWC computed
   const int HWL = ROWS ? a.HR * a.W : a.HW, HWC = ROWS ? a.HC * a.W : a.HW;
-  const int NPX = a.T * HWL;
+  const int NPX = T * HWL;
   const int BUFB = (NPX + ZERO_PIX) * PIXB;
   uint8_t* V0 = lds;
   uint8_t* V1 = V0 + BUFB;
@@ -484,10 +506,10 @@ __global__ __launch_bounds__(64 * NWAVE) void convar_fwd_kernel(FwdArgs a) {
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int NW = blockDim.x >> 6;
   const int n16 = lane & 15, g = lane >> 4;
-  const int H = a.H, W = a.W, HW = a.HW, T = a.T;
+  const int H = a.H, W = a.W, HW = a.HW;
   const int HR = ROWS ? a.HR : H, ROW0 = ROWS ? a.ROW0 : 0;
   const int gofs = ROWS ? (a.R0 - ROW0) * W : 0;  // global index of a configuration's LDS pixel 0
-  const int ntiles = npix >> 4;
+  const int ntiles = (PREC == FK_PREC_FP32 ? a.npix : T * HWC + 15) >> 4;
   const int nt = (ntiles > wave) ? (ntiles - wave + NW - 1) / NW : 0;
 
   int pix[MAXT], pi[MAXT], pj[MAXT];
@@ -539,13 +561,7 @@ __global__ __launch_bounds__(64 * NWAVE) void convar_fwd_kernel(FwdArgs a) {
     reinterpret_cast<uint32_t*>(H1 + NPX * PIXB)[z] = 0u;
   }
 
-  int64_t M = a.m_dev ? *a.m_dev : a.m_count;
-  int64_t m0 = 0;
-  if (a.m_range) {
-    m0 = a.m_range[0];
-    M = a.m_range[1] - m0;
-  }
-  if (M > a.m_count) M = a.m_count;
+  if constexpr (PREC == FK_PREC_FP32) M = count(m0);
   const int64_t ngroups = (M + T - 1) / T;
   const int nb = a.nblocks;
   const frag* wall = reinterpret_cast<const frag*>(a.w);
@@ -783,7 +799,8 @@ __global__ __launch_bounds__(64 * NWAVE) void convar_fwd_kernel(FwdArgs a) {
               if (u < nt) valu_v(u, acc[u]);
             hh.load_bias(bias + C, g);
           } else {
-            conv_pass<PREC, C, MAXT, 0, MT>(acc, Vin, wall + lay.off_v(blk) * 64, toff, lane, hv);
+            if (MAXT > 1 || nt > 0)
+              conv_pass<PREC, C, MAXT, 0, MT>(acc, Vin, wall + lay.off_v(blk) * 64, toff, lane, hv);
             hh.load(wall + lay.off_h(blk) * 64, bias + C, lane, g);
           }
 #pragma unroll
@@ -801,7 +818,8 @@ __global__ __launch_bounds__(64 * NWAVE) void convar_fwd_kernel(FwdArgs a) {
             for (int u = 0; u < MAXT; ++u)
               if (u < nt) valu_h(u, acc[u]);
           } else {
-            conv_pass<PREC, C, MAXT, 1, MT>(acc, Hin, wall + lay.off_h(blk) * 64, toff, lane, hh);
+            if (MAXT > 1 || nt > 0)
+              conv_pass<PREC, C, MAXT, 1, MT>(acc, Hin, wall + lay.off_h(blk) * 64, toff, lane, hh);
           }
           hc.load(wall + lay.off_c(blk) * 64, bias + 3 * C, lane, g);
 #pragma unroll
@@ -902,7 +920,8 @@ __global__ __launch_bounds__(64 * NWAVE) void convar_fwd_kernel(FwdArgs a) {
         for (int u = 0; u < MAXT; ++u)
 #pragma unroll
           for (int mt = 0; mt < MT; ++mt) acc[u][mt] = hc.bias[mt];
-        conv_pass<PREC, C, MAXT, 2, MT>(acc, CAT, wall + lay.off_c(blk) * 64, toff, lane, hc);
+        if (MAXT > 1 || nt > 0)
+          conv_pass<PREC, C, MAXT, 2, MT>(acc, CAT, wall + lay.off_c(blk) * 64, toff, lane, hc);
         // the next block's vertical pass (block 0 of the next group: bias only)
         if (blk + 1 < nb) hv.load(wall + lay.off_v(blk + 1) * 64, a.aux + lay.aux_bias(blk + 1), lane, g);
         else hv.load_bias(a.aux + lay.aux_bias(0), g);
@@ -974,6 +993,7 @@ __global__ __launch_bounds__(64 * NWAVE) void convar_fwd_kernel(FwdArgs a) {
 struct FwdPlan {
   int T, npix, maxt, nwave;
   size_t lds;
+  int64_t slots;  // workgroups that run at once with the largest tile
 };
 
 // workgroups that fit a CU's 160 KB of LDS (dynamic + static)
@@ -982,14 +1002,12 @@ inline int fwd_per_cu(const FwdPlan& pl) {
   return n > 0 ? n : 1;
 }
 
-// persistent grid: CU count x workgroups per CU, at most one per group
+// persistent grid: CU count x workgroups per CU, at most one per
+// configuration (per group where the count is not read on the device)
 inline int64_t fwd_grid(const FwdArgs& a, const FwdPlan& pl) {
-  const int64_t ngroups = (a.m_count + pl.T - 1) / pl.T;
-  const int per_cu = fwd_per_cu(pl);
-  int64_t grid = (int64_t)device_cu_count() * per_cu;
-  if (grid > ngroups) grid = ngroups;
-  if (grid < 1) grid = 1;
-  return grid;
+  const int64_t n = a.m_dev || a.m_range ? a.m_count : (a.m_count + pl.T - 1) / pl.T;
+  const int64_t grid = pl.slots < n ? pl.slots : n;
+  return grid < 1 ? 1 : grid;
 }
 
 template <int PREC, int C, int MAXT, int ACT, int NWAVE, int SCHED, bool HG, bool ROWS>
@@ -1008,6 +1026,16 @@ int launch_fwd(const FwdArgs& a, const FwdPlan& pl, hipStream_t s) {
 template <int PREC, int C, int NW, int SCHED, bool HG, bool ROWS>
 int launch_variant(const FwdArgs& a, const FwdPlan& pl, int act, hipStream_t s) {
   constexpr int LO = NW == 4 ? 4 : 2, HI = NW == 4 ? 8 : 4;
+  // FP32: waves of at most one tile.  Its MFMAs take 32 cycles, so tiles that are
+  // not there cost as much as the others, and so do waves without any (one
+  // 10x10 C 32 depth 20 configuration 1.07 -> 0.66 ms, 16 of 4x4 C 16 depth 5
+  // 60 -> 31 us, 300 of 3x3 C 64 0.97 -> 0.32 ms).  In 16 bits they hide behind
+  // the operands.
+  if constexpr (PREC == FK_PREC_FP32 && NW == 8 && SCHED == 0 && !ROWS) {
+    if (pl.maxt == 1)
+      return act == FK_ACT_ELU ? launch_fwd<PREC, C, 1, FK_ACT_ELU, NW, SCHED, HG, ROWS>(a, pl, s)
+                               : launch_fwd<PREC, C, 1, FK_ACT_RELU, NW, SCHED, HG, ROWS>(a, pl, s);
+  }
   if (pl.maxt <= LO)
     return act == FK_ACT_ELU ? launch_fwd<PREC, C, LO, FK_ACT_ELU, NW, SCHED, HG, ROWS>(a, pl, s)
                              : launch_fwd<PREC, C, LO, FK_ACT_RELU, NW, SCHED, HG, ROWS>(a, pl, s);

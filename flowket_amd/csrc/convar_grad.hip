@@ -29,7 +29,7 @@
 // block, four waves) the matrix cores were busy a quarter of the time.
 // Measured, VJP / JVP / O in ms, before -> now: 10x10 depth 20 C 32, 64
 // samples 5.86 / 3.81 / 9.21 -> 1.91 / 1.45 / 3.08; 2048 samples 25.4 / 19.7 /
-// 36.1 -> 15.4 / 11.5 / 24.8; 20x20 depth 24 C 64,
+// samples 5.86 / 3.81 / 9.21 / 11.5 / 24.8; 20x20 depth 24 C 64,
 // 128 samples 88.6 / 56.3 / 155.9 -> 27.6 / 22.5 / 45.2; 4x4 depth 5 C 32, 1024
 // samples 1.54 / 0.66 / 1.23 -> 0.65 / 0.21 / 0.74.
 #include "convar_bwd.h"
@@ -38,10 +38,6 @@ namespace fk {
 
 namespace {
 
-// The units of a phase are one list, taken by the waves from a counter in LDS:
-// a wave's first unit is its number, the next come from the counter, so waves
-// that drew short units take more.  Which wave computes a unit does not change
-// it: results are deterministic.
 struct Lane {
   int l16, kk;  // this lane's column and contraction group (lane l16 + 16 kk)
   // (opaque: what follows from it is computed where it is used, not kept in
@@ -51,6 +47,10 @@ struct Lane {
   }
 };
 
+// The units of a phase are one list, taken by the waves from a counter in LDS:
+// a wave's first unit is its number, the next come from the counter, so waves
+// that drew short units take more.  Which wave computes a unit does not change
+// it: results are deterministic.
 struct Work {
   int* q;  // 4 counters, one per phase (modulo 4)
   int phase, cur;

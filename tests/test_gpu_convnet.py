@@ -287,3 +287,28 @@ def test_schedule_is_per_network(rng):
             assert torch.equal(b.log_psi(x), before)
     finally:
         autotune.set_schedule(a, _lib.FK_PREC_BF16, -1)
+
+
+@pytest.mark.parametrize('shape,depth,C,act,prec', [((4, 4), 5, 16, 'elu', 'fp32'), ((10, 10), 4, 32, 'relu', 'fp32'),
+                                                    ((5, 7), 4, 20, 'relu', 'fp16'), ((3, 3), 3, 64, 'elu', 'bf16'),
+                                                    ((14, 14), 3, 64, 'relu', 'fp32')])
+def test_tiles_of_every_batch_give_the_same_bits(rng, shape, depth, C, act, prec):
+    """How many configurations share a workgroup follows from the batch (one
+    a workgroup, a round more or less, the largest tile); a configuration's
+    log psi does not.  Local energies read the counts on the device; theirs
+    differ by the FP32 rounding of log psi at most (row reuse may differ)."""
+    gpu_banner(f'tiles by batch shape={shape} depth={depth} C={C} {prec}')
+    import flowket_amd as fk
+    m = _machine(shape, depth, C, act, prec)
+    x = torch.as_tensor(rng.choice([-1, 1], size=(9001,) + shape).astype(np.int8)).to(m.device)
+    full = m.log_psi(x)
+    for n in (1, 2, 7, 255, 256, 257, 511, 513, 1025, 3000, 8193):
+        assert torch.equal(torch.view_as_real(m.log_psi(x[:n])), torch.view_as_real(full[:n])), n
+    ref = ocn.log_psi(_oracle_params(m), x[-3:].cpu().numpy(), depth, activation=act)
+    _check_logpsi(full[-3:], ref, RTOL[prec])
+    if prec == 'fp32':
+        obs = fk.Observable(fk.Ising(h=1.0, hilbert_state_shape=shape, pbc=False))
+        e = obs.local_values(m, x[:300])
+        for n in (1, 40):
+            d = (obs.local_values(m, x[:n]) - e[:n]).abs()
+            assert (d <= 1e-4 * (1 + e[:n].abs())).all()
