@@ -30,7 +30,8 @@ struct BwdArgs {
   int64_t P;
   int64_t ld;           // row stride of o_re / o_im (>= P)
   const float* cot;     // GRAD_VJP: (batch, 2) cotangents of (Re, Im) log psi
-  float* partial;       // GRAD_VJP: (gridDim.x, P) per-workgroup partial gradients
+  float* partial;       // GRAD_VJP: partial gradients, rows of P floats
+  int64_t run;          // convar_grad.hip: samples of a workgroup that share a partial row
   const float* tangent; // JVP: direction, P floats
   float* jvp;           // JVP: (batch, 2) output
   const float* kt;      // the conv kernels transposed (transpose_kernels_kernel), P floats

@@ -916,8 +916,9 @@ __device__ __forceinline__ void block_sums(float (&v)[NV], float* red) {  // red
 
 // MODE GRAD_O: one workgroup per sample, two backward passes (the cotangents
 // of Re and Im log psi) into its rows of O_re and O_im.  GRAD_VJP: a
-// persistent grid; each workgroup adds its samples' cot_re d Re log psi +
-// cot_im d Im log psi to its own partial gradient row.  GRAD_JVP: forward mode.
+// persistent grid; cot_re d Re log psi + cot_im d Im log psi of a workgroup's
+// samples, run by run (a.run samples), is summed in partial rows of its own: run
+// r of workgroup w in row r gridDim.x + w.  GRAD_JVP: forward mode.
 template <int C_, int ACT, int MODE, bool RES_, int NT>
 __global__ __launch_bounds__(NT, NT == 1024 ? 4 : 2) void convar_grad_kernel3(BwdArgs a) {
   constexpr bool TAN = MODE == GRAD_JVP;
@@ -955,10 +956,8 @@ __global__ __launch_bounds__(NT, NT == 1024 ? 4 : 2) void convar_grad_kernel3(Bw
   }
   build_tables(ftab, itab, a.H, a.W);
   Work wk{s_q, 0, 0};
-  float* part = nullptr;
-  if constexpr (MODE == GRAD_VJP) {
-    part = a.partial + (int64_t)blockIdx.x * a.P;
-  }
+  float* part = MODE == GRAD_VJP ? a.partial + (int64_t)blockIdx.x * a.P : nullptr;
+  int64_t k = 0;  // the sample's number in its run
   const int64_t ho = head_offset(nb, C);
   for (int64_t b = blockIdx.x; b < a.batch; b += gridDim.x) {
     for (int q = threadIdx.x; q < HW; q += NT) x.ws[q] = (float)a.spins[b * HW + q];
@@ -1016,7 +1015,7 @@ __global__ __launch_bounds__(NT, NT == 1024 ? 4 : 2) void convar_grad_kernel3(Bw
       else __syncthreads();
       if constexpr (!TAN) {
         float* O = MODE == GRAD_VJP ? part : (pass == 0 ? a.o_re : a.o_im) + b * a.ld;
-        backward<S, ACT, MODE == GRAD_VJP>(wk, x, dz, O, b != blockIdx.x);
+        backward<S, ACT, MODE == GRAD_VJP>(wk, x, dz, O, k > 0);
       }
     }
     if (threadIdx.x == 0) {
@@ -1027,6 +1026,12 @@ __global__ __launch_bounds__(NT, NT == 1024 ? 4 : 2) void convar_grad_kernel3(Bw
       if constexpr (TAN) {
         a.jvp[2 * b] = sums[2];
         a.jvp[2 * b + 1] = sums[3];
+      }
+    }
+    if constexpr (MODE == GRAD_VJP) {
+      if (++k == a.run) {
+        k = 0;
+        part += gridDim.x * a.P;
       }
     }
     __syncthreads();

@@ -253,6 +253,30 @@ def test_gradient_kernels_over_tiles_and_grids(rng, shape, depth, C, act, B):
             assert (got[:, :P] - want).abs().max().item() < 1e-5 * np.abs(O).max()
 
 
+@pytest.mark.parametrize('shape,C,per_cu', [((4, 4), 32, 4), ((9, 8), 64, 3)])
+def test_vjp_adds_few_samples_in_fp32(rng, shape, C, per_cu):
+    """The batched VJP adds samples in FP32 in 4 (or, where a sample's tensors
+    are not staged in LDS, 3) partial rows a CU and the rows in FP64, so up to
+    that many samples a CU are added in FP64 alone.  As many samples as CUs are
+    one configuration with cotangents of 2^20 and -2^20 in turn, which cancel
+    exactly; the others added to them in FP32 would lose 2^-4 of their size.
+    The bound is that of the tests above."""
+    import flowket_amd as fk
+    cu = torch.cuda.get_device_properties(0).multi_processor_count
+    rows = per_cu * cu
+    m = fk.ConvNetAutoregressive2D(shape, depth=2, num_of_channels=C, activation='elu', weights_normalization=False,
+                                   precision='fp32', seed=8)
+    s = rng.choice([-1, 1], size=(rows,) + shape).astype(np.int8)
+    u = rng.normal(size=(rows, 2))
+    s[:cu] = s[0]
+    u[0:cu:2], u[1:cu:2] = 2.0 ** 20, -2.0 ** 20
+    got = m.vjp(s, torch.as_tensor(u, dtype=torch.float32)).double().cpu().numpy()
+    o_re, o_im, _ = m.per_sample_gradients(s[cu:])
+    w = torch.as_tensor(u[cu:], device=m.device)
+    ref = (o_re.T.double() @ w[:, 0] + o_im.T.double() @ w[:, 1]).cpu().numpy()
+    assert np.abs(got - ref).max() < 2e-5 * np.abs(ref).max()
+
+
 @pytest.mark.parametrize('B,P', [(37, 1000), (37, 1001), (5, 4)])
 def test_sr_products_c_abi(rng, B, P):
     """fk_o_times_v / fk_oh_times_u on random O against dense float64 algebra,
