@@ -25,6 +25,19 @@ def num_causal_blocks(depth):
     return 2 + 2 * max(depth - 2, 0)
 
 
+def _plain_storage(t, n):
+    """Whether t is n contiguous float32 values on the current GPU that a
+    kernel may read in place of an expression in torch: nothing records,
+    differentiates or transforms operations on it (autograd, forward-mode
+    duals, torch.func wrappers, tensor subclasses, dispatch modes, tracing)."""
+    return (type(t) in (torch.Tensor, torch.nn.Parameter) and t.numel() == n and t.dtype == torch.float32 and
+            t.device.type == 'cuda' and t.device.index == torch.cuda.current_device() and
+            not (torch.is_grad_enabled() and t.requires_grad) and
+            not torch._C._functorch.is_functorch_wrapped_tensor(t) and t.is_contiguous() and
+            torch.autograd.forward_ad.unpack_dual(t).tangent is None and
+            not torch._C._len_torch_dispatch_stack() and not torch.jit.is_tracing())
+
+
 def layer_shapes(depth, channels, kernel_size=3):
     """(kernel shape, bias shape) of every convolution in network order:
     per causal block vconv, hconv, x1x1, y1x1, h3conv
@@ -192,10 +205,13 @@ class ConvNetAutoregressive2D:
     def effective_params(self):
         """The flat kernel/bias vector the network actually uses: the raw
         parameters, or with weight normalisation kernel = l2_normalize(v)
-        * exp(g) per output channel (wrappers.py:123-135)."""
+        * exp(g) per output channel (wrappers.py:123-135).  One launch
+        (fk_wn_effective) where both are plain device tensors, else an expression
+        in torch, so that autograd and function transforms see it."""
         if not self.weights_normalization:
             return self.params
-        if self.device.type == 'cuda':
+        if (self.device.type == 'cuda' and _plain_storage(self.params, self.n_params) and
+                _plain_storage(self.wn_g, self.n_trainable - self.n_params)):
             tab, nl, mc = self._wn_table()
             eff = torch.empty(self.n_params, dtype=torch.float32, device=self.device)
             _lib.call('fk_wn_effective', _lib.ptr(self.params), _lib.ptr(self.wn_g), _lib.ptr(tab), nl, mc,

@@ -304,3 +304,44 @@ def test_wn_effective_kernels(depth, channels, exp_norm):
         np.testing.assert_allclose(got[off:off + nk], ref, rtol=2.4e-7, atol=0)
         np.testing.assert_array_equal(got[off + nk:off + nk + bs[0]], p[off + nk:off + nk + bs[0]])
         off += nk + bs[0]
+
+
+def _wn_machine(device=None):
+    import flowket_amd as fk
+    return fk.ConvNetAutoregressive2D((3, 3), depth=3, num_of_channels=6, weights_normalization=True, seed=9,
+                                      device=device)
+
+
+@pytest.mark.gpu
+def test_effective_params_follow_torch_transforms(rng):
+    """effective_params is an expression of params and wn_g for autograd,
+    forward mode, torch.func and other layouts and types, on the GPU as on the
+    CPU.  FP32 sums of up to 54 squares and a dot of 54 products: 1e-5."""
+    from torch.autograd import forward_ad
+    cot = torch.as_tensor(rng.normal(size=_wn_machine('cpu').n_params), dtype=torch.float32)
+    step = torch.as_tensor(rng.normal(size=(2, cot.numel())), dtype=torch.float32)
+    got = {}
+    for device in ('cpu', 'cuda'):
+        m = _wn_machine(device)
+        p, g, c, t = m.params.clone(), m.wn_g.clone(), cot.to(device), step.to(device)
+
+        def effective(params):
+            m.params = params
+            return m.effective_params()
+
+        out = {'plain': effective(p), 'strided': effective(torch.stack([p, p], 1)[:, 0]),
+               'double': effective(p.double()).float()}
+        leaf = p.clone().requires_grad_(True)
+        m.wn_g = g.clone().requires_grad_(True)
+        out['grad'], out['grad_g'] = torch.autograd.grad(effective(leaf) @ c, (leaf, m.wn_g))
+        out['grad_g_only'], = torch.autograd.grad(effective(p) @ c, m.wn_g)
+        with torch.no_grad():
+            assert not effective(leaf).requires_grad
+        m.wn_g = g
+        with forward_ad.dual_level():
+            out['dual'] = forward_ad.unpack_dual(effective(forward_ad.make_dual(p, t[0]))).tangent
+        out['func'] = torch.func.grad(lambda x: effective(x) @ c)(p)
+        out['vmap'] = torch.func.vmap(effective)(p + t)
+        got[device] = {k: v.detach().cpu().double() for k, v in out.items()}
+    for k, ref in got['cpu'].items():
+        assert (got['cuda'][k] - ref).abs().max() < 1e-5 * ref.abs().max(), k
