@@ -104,6 +104,8 @@ class ConvNetAutoregressive2D:
         self._packs = {}
         self._maps = {}
         self._fws = {}
+        if self.weights_normalization:
+            self._wn_table()  # (a copy to the device: not while a graph is captured)
         self.conditional_log_probs_model = _ConditionalLogProbsModel(self)
 
     # ------------------------------------------------------------------ params

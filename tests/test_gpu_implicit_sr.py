@@ -345,3 +345,20 @@ def test_effective_params_follow_torch_transforms(rng):
         got[device] = {k: v.detach().cpu().double() for k, v in out.items()}
     for k, ref in got['cpu'].items():
         assert (got['cuda'][k] - ref).abs().max() < 1e-5 * ref.abs().max(), k
+
+
+@pytest.mark.gpu
+def test_effective_params_first_called_under_capture():
+    """Replays after updates of the parameters, against the eager result."""
+    m, eager = _wn_machine('cuda'), _wn_machine('cuda')
+    g = torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(g):
+        out = m.effective_params()
+    for k in range(3):
+        p = m.params.cpu() * (1.0 + 0.1 * k)
+        m.set_params(p)
+        eager.set_params(p)
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, eager.effective_params())

@@ -80,3 +80,13 @@ def test_effective_kernel_of_the_loaded_weights():
     kshape = m.shapes[0][0]
     k0 = eff[:int(np.prod(kshape))].reshape(kshape)
     assert np.allclose(np.sqrt((k0 ** 2).sum(axis=(0, 1, 2))), np.exp(fx['g'][:kshape[3]]), rtol=1e-5)
+
+
+def test_wn_table_is_made_with_the_machine(monkeypatch):
+    """Nothing is copied to the device by the first call of effective_params,
+    which may be under capture."""
+    import flowket_amd as fk
+    import flowket_amd.machines as machines
+    m = fk.ConvNetAutoregressive2D((3, 3), depth=3, num_of_channels=6, weights_normalization=True, device='cpu')
+    monkeypatch.setattr(machines.torch, 'as_tensor', lambda *a, **k: pytest.fail('a copy'))
+    assert m._wn_table()[1] == len(m.shapes) - 1
