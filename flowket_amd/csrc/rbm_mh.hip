@@ -248,21 +248,24 @@ struct MhArgs {
   int32_t* nonfinite;      // set to 1 when a proposal's log psi is not finite (or null)
 };
 
-// One workgroup per chain, a wave per 64 hidden units (M <= 64 * NW), one
-// unit per lane.  A step is a serial chain -- theta', lncosh, the sum over
-// the units, the decision -- so it is latency that bounds a chain: all units
-// in one wave took the lncosh of four units per lane in turn.  1024 chains x
-// 319 exchange proposals of the 8x8 alpha-4 RBM: 921 us in one wave, 480 in
-// four with the proposals drawn 64 at a time (four waves that each drew every
-// proposal were no faster than one).
+// One workgroup of NW waves per chain, HPL hidden units a lane (M <= 64 NW HPL).
+// A step is a serial chain -- theta', lncosh, the sum over the units, the
+// decision -- so while the chip is not full it is latency that bounds a chain,
+// and a wave per 64 units is the fastest (1024 chains x 319 exchange proposals
+// of the 8x8 alpha-4 RBM: 921 us in one wave, 480 in four with the proposals
+// drawn 64 at a time).  Once it is full every wave's own instructions count (the
+// draws, the sum, the decision), and fewer waves with more units are: with 191
+// exchange / local proposals 2048 chains take 554 / 715 us in four waves and 421
+// / 591 in two, 16384 chains 3.56 / 4.72 ms in four and 1.90 / 3.00 in one.
 // The waves exchange their units' terms through LDS (double-buffered, one
 // barrier a step); every wave then adds a lane's terms in unit order and
 // reduces over the lanes, so all reach the same decision, the one a single
-// wave would.
-template <int NW>
-__global__ __launch_bounds__(64 * NW) void mh_rbm_kernel(MhArgs a) {
+// wave would: chains do not depend on NW and HPL.
+template <int NW, int HPL>
+__global__ __launch_bounds__(64 * NW, 4) void mh_rbm_kernel(MhArgs a) {
+  constexpr int NU = NW * HPL;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  __shared__ float s_part[2][NW][64];
+  __shared__ float s_part[2][NW > 1 ? NU : 1][64];
   const int64_t ch = blockIdx.x;
   if (ch >= a.chains) return;
   const RbmParams& p = a.p;
@@ -270,23 +273,33 @@ __global__ __launch_bounds__(64 * NW) void mh_rbm_kernel(MhArgs a) {
   extern __shared__ int8_t s_state[];  // N spins of this chain
   for (int j = threadIdx.x; j < N; j += 64 * NW) s_state[j] = a.state[ch * N + j];
   __syncthreads();
-  const int h = (int)threadIdx.x;
-  const bool unit = h < M;
-  float tr = 0.0f, ti = 0.0f;
-  auto theta = [&]() {  // from the state
-    tr = p.b_re[h];
-    ti = -p.b_im[h];
+  int h[HPL];
+  bool unit[HPL];
+#pragma unroll
+  for (int u = 0; u < HPL; ++u) {
+    h[u] = 64 * (wave * HPL + u) + lane;
+    unit[u] = h[u] < M;
+  }
+  float tr[HPL], ti[HPL];
+  auto theta = [&](int u) {  // from the state
+    tr[u] = p.b_re[h[u]];
+    ti[u] = -p.b_im[h[u]];
 #pragma unroll 4
     for (int j = 0; j < N; ++j) {
       const float s = (float)s_state[j];
-      tr += p.w_re[(int64_t)j * M + h] * s;
-      ti -= p.w_im[(int64_t)j * M + h] * s;
+      tr[u] += p.w_re[(int64_t)j * M + h[u]] * s;
+      ti[u] -= p.w_im[(int64_t)j * M + h[u]] * s;
     }
   };
-  if (unit) theta();
   // Re lncosh(theta) of the current state, kept with theta (recomputed
   // only where theta changes)
-  float lc = unit ? lncosh_re(tr, ti) : 0.0f;
+  float lc[HPL];
+#pragma unroll
+  for (int u = 0; u < HPL; ++u) {
+    tr[u] = ti[u] = 0.0f;
+    if (unit[u]) theta(u);
+    lc[u] = unit[u] ? lncosh_re(tr[u], ti[u]) : 0.0f;
+  }
   const int64_t total = a.n_burn + a.n_record * (a.unused + 1);
   int64_t acc = 0;
   // The proposal of a step: sites (j2 = -1 for local moves) and uniform, from
@@ -323,7 +336,7 @@ __global__ __launch_bounds__(64 * NW) void mh_rbm_kernel(MhArgs a) {
   };
   int cj1 = 0, cj2 = -1;
   double cu = 0.0;
-  float pw1r = 0.0f, pw1i = 0.0f, pw2r = 0.0f, pw2i = 0.0f;
+  float pw1r[HPL] = {}, pw1i[HPL] = {}, pw2r[HPL] = {}, pw2i[HPL] = {};
   float pa1 = 0.0f, pa2 = 0.0f;
   auto prefetch = [&](int64_t st) {
     const int l = (int)(st & 63);
@@ -333,11 +346,14 @@ __global__ __launch_bounds__(64 * NW) void mh_rbm_kernel(MhArgs a) {
     cu = __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(du), l),
                           __builtin_amdgcn_readlane(__double2loint(du), l));
     const int jb = cj2 >= 0 ? cj2 : cj1;
-    if (unit) {
-      pw1r = p.w_re[(int64_t)cj1 * M + h];
-      pw1i = p.w_im[(int64_t)cj1 * M + h];
-      pw2r = p.w_re[(int64_t)jb * M + h];
-      pw2i = p.w_im[(int64_t)jb * M + h];
+#pragma unroll
+    for (int u = 0; u < HPL; ++u) {
+      if (unit[u]) {
+        pw1r[u] = p.w_re[(int64_t)cj1 * M + h[u]];
+        pw1i[u] = p.w_im[(int64_t)cj1 * M + h[u]];
+        pw2r[u] = p.w_re[(int64_t)jb * M + h[u]];
+        pw2i[u] = p.w_im[(int64_t)jb * M + h[u]];
+      }
     }
     pa1 = p.a_re[cj1];
     pa2 = p.a_re[jb];
@@ -348,15 +364,30 @@ __global__ __launch_bounds__(64 * NW) void mh_rbm_kernel(MhArgs a) {
     if (step > 0 && (step & 255) == 0) {
       // refresh theta from the state (bounds the drift of the FP32
       // incremental updates)
-      if (unit) {
-        theta();
-        lc = lncosh_re(tr, ti);
+      auto refresh = [&](int u) {
+        if (unit[u]) {
+          theta(u);
+          lc[u] = lncosh_re(tr[u], ti[u]);
+        }
+      };
+      if constexpr (HPL == 1) {  // (a loop of one trip took 11 scalar registers more, spilled)
+        refresh(0);
+      } else {
+#pragma unroll
+        for (int u = 0; u < HPL; ++u) refresh(u);
       }
     }
     // ---- proposal: drawn (and its weight rows requested) one step ahead
     const int j1 = cj1, j2 = cj2;
-    const double u = cu;
-    const float w1r = pw1r, w1i = pw1i, w2r = pw2r, w2i = pw2i;
+    const double uniform = cu;
+    float w1r[HPL], w1i[HPL], w2r[HPL], w2i[HPL];
+#pragma unroll
+    for (int u = 0; u < HPL; ++u) {
+      w1r[u] = pw1r[u];
+      w1i[u] = pw1i[u];
+      w2r[u] = pw2r[u];
+      w2i[u] = pw2i[u];
+    }
     const float a1 = pa1, a2 = pa2;
     if (step + 1 < total) prefetch(step + 1);
     // sites that change: local -> j1; exchange -> j1 and j2 if they differ
@@ -368,29 +399,40 @@ __global__ __launch_bounds__(64 * NW) void mh_rbm_kernel(MhArgs a) {
       flip2 = flip1;
     }
     float dre = 0.0f;
-    float nr = tr, ni = ti, nl = lc;
+    float nr[HPL], ni[HPL], nl[HPL];
+#pragma unroll
+    for (int u = 0; u < HPL; ++u) {
+      nr[u] = tr[u];
+      ni[u] = ti[u];
+      nl[u] = lc[u];
+    }
     if (flip1) {  // uniform over the workgroup, as every branch of the step
       const float s2 = flip2 ? (float)s_state[j2] : 0.0f;
-      if (unit) {
-        nr -= 2.0f * s1 * w1r;
-        ni += 2.0f * s1 * w1i;
-        if (flip2) {
-          nr -= 2.0f * s2 * w2r;
-          ni += 2.0f * s2 * w2i;
+#pragma unroll
+      for (int u = 0; u < HPL; ++u) {
+        if (unit[u]) {
+          nr[u] -= 2.0f * s1 * w1r[u];
+          ni[u] += 2.0f * s1 * w1i[u];
+          if (flip2) {
+            nr[u] -= 2.0f * s2 * w2r[u];
+            ni[u] += 2.0f * s2 * w2i[u];
+          }
+          nl[u] = lncosh_re(nr[u], ni[u]);
         }
-        nl = lncosh_re(nr, ni);
       }
       if constexpr (NW > 1) {
         // (a wave writes a buffer again two exchanges later, after the barrier
         // of the one between, which every reader of this one has reached)
         float(*part)[64] = s_part[buf];
         buf ^= 1;
-        part[wave][lane] = unit ? nl - lc : 0.0f;
+#pragma unroll
+        for (int u = 0; u < HPL; ++u) part[wave * HPL + u][lane] = unit[u] ? nl[u] - lc[u] : 0.0f;
         __syncthreads();
 #pragma unroll
-        for (int k = 0; k < NW; ++k) dre += part[k][lane];
+        for (int k = 0; k < NU; ++k) dre += part[k][lane];
       } else {
-        dre += unit ? nl - lc : 0.0f;
+#pragma unroll
+        for (int u = 0; u < HPL; ++u) dre += unit[u] ? nl[u] - lc[u] : 0.0f;
       }
       dre = wave_sum(dre);
       dre += -2.0f * s1 * a1;
@@ -402,12 +444,15 @@ __global__ __launch_bounds__(64 * NW) void mh_rbm_kernel(MhArgs a) {
     const bool finite = isfinite(dre);
     if (!finite && a.nonfinite && threadIdx.x == 0) a.nonfinite[0] = 1;
     const float lr = fminf(2.0f * dre, 0.0f);
-    const bool accept = finite && (double)expf(lr) > u;
+    const bool accept = finite && (double)expf(lr) > uniform;
     if (accept) {
       if (flip1) {
-        tr = nr;
-        ti = ni;
-        lc = nl;
+#pragma unroll
+        for (int u = 0; u < HPL; ++u) {
+          tr[u] = nr[u];
+          ti[u] = ni[u];
+          lc[u] = nl[u];
+        }
         // every wave has read the state by the exchange's barrier above
         if (NW == 1) __syncthreads();
         if (threadIdx.x == 0) {
@@ -436,15 +481,19 @@ __global__ __launch_bounds__(64 * NW) void mh_rbm_kernel(MhArgs a) {
   if (threadIdx.x == 0) a.accepts[ch] = acc;
   if (!a.logpsi) return;
   // final log psi from theta, a lane's units in order
-  __shared__ float s_fin[NW][2][64];
-  if (unit) lncosh(tr, ti, tr, ti);
-  s_fin[wave][0][lane] = unit ? tr : 0.0f;
-  s_fin[wave][1][lane] = unit ? ti : 0.0f;
+  __shared__ float s_fin[NU][2][64];
+#pragma unroll
+  for (int u = 0; u < HPL; ++u) {
+    float r = 0.0f, i = 0.0f;
+    if (unit[u]) lncosh(tr[u], ti[u], r, i);
+    s_fin[wave * HPL + u][0][lane] = r;
+    s_fin[wave * HPL + u][1][lane] = i;
+  }
   __syncthreads();
   if (wave > 0) return;
   float lr = 0.0f, li = 0.0f;
 #pragma unroll
-  for (int k = 0; k < NW; ++k) {
+  for (int k = 0; k < NU; ++k) {
     if (lane + 64 * k < M) {
       lr += s_fin[k][0][lane];
       li += s_fin[k][1][lane];
@@ -655,10 +704,20 @@ int fk_mh_rbm(const float* w_re, const float* w_im, const float* b_re, const flo
   a.r_u = r_u;
   a.seed = seed;
   a.nonfinite = nonfinite;
+  if (n_hidden > 512) {
+    set_error("fk_mh_rbm: at most 512 hidden units");
+    return FK_ERR_UNSUPPORTED;
+  }
   const size_t lds = (size_t)((n_visible + 15) & ~15);
   hipStream_t s = (hipStream_t)stream;
-  const int waves = (n_hidden + 63) / 64;
-  auto launch = [&](auto kern, int nw) -> int {
+  const int units = n_hidden <= 64 ? 1 : n_hidden <= 128 ? 2 : n_hidden <= 256 ? 4 : 8;  // of 64
+  // a wave per unit while that leaves at most four waves a SIMD, then fewer of up
+  // to four units (128 units: the two forms cross at about 1200 chains and differ
+  // by 6 % at 2048; 256 units: at 1000 and 2300; 400 to 512: at 450 and 1800;
+  // eight units a lane are slower than four everywhere)
+  int nw = units;
+  while (nw > 1 && units / nw < 4 && chains * nw > 16LL * device_cu_count()) nw /= 2;
+  auto launch = [&](auto kern) -> int {
     // the state and the waves' exchange buffers together may pass the 64 KB
     // that a launch gets unasked
     if (lds > 48 * 1024)
@@ -668,12 +727,11 @@ int fk_mh_rbm(const float* w_re, const float* w_im, const float* b_re, const flo
     FK_CHECK_LAUNCH();
     return FK_OK;
   };
-  if (waves <= 1) return launch(mh_rbm_kernel<1>, 1);
-  if (waves <= 2) return launch(mh_rbm_kernel<2>, 2);
-  if (waves <= 4) return launch(mh_rbm_kernel<4>, 4);
-  if (waves <= 8) return launch(mh_rbm_kernel<8>, 8);
-  set_error("fk_mh_rbm: at most 512 hidden units");
-  return FK_ERR_UNSUPPORTED;
+  if (units == 1) return launch(mh_rbm_kernel<1, 1>);
+  if (units == 2) return nw == 2 ? launch(mh_rbm_kernel<2, 1>) : launch(mh_rbm_kernel<1, 2>);
+  if (units == 4)
+    return nw == 4 ? launch(mh_rbm_kernel<4, 1>) : nw == 2 ? launch(mh_rbm_kernel<2, 2>) : launch(mh_rbm_kernel<1, 4>);
+  return nw == 8 ? launch(mh_rbm_kernel<8, 1>) : nw == 4 ? launch(mh_rbm_kernel<4, 2>) : launch(mh_rbm_kernel<2, 4>);
 }
 
 int fk_rbm_grad(const float* w_re, const float* w_im, const float* b_re, const float* b_im, const float* a_re,

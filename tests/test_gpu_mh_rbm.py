@@ -245,3 +245,58 @@ def test_rbm_log_psi_many_configurations(rng, n, alpha):
     assert torch.equal(torch.cat([got[:9], got[-9:]]), one)
     ref = _oracle_lp(m, s[-9:].numpy())
     assert np.abs(got[-9:].real.cpu().numpy() - ref.real).max() / (np.abs(ref.real).max() + 1) < 1e-5
+
+
+def _mh_rbm(m, shape, kind, start, sites, moves, us, n_burn, spc, unused):
+    """fk_mh_rbm on injected randomness: samples, final states, accepts and
+    final log psi."""
+    from flowket_amd import _lib
+    C, n = start.shape
+    state = start.clone()
+    out = torch.empty((C, spc, n), dtype=torch.int8, device='cuda')
+    accepts = torch.empty(C, dtype=torch.int64, device='cuda')
+    logpsi = torch.empty((C, 2), device='cuda')
+    flag = torch.zeros(1, dtype=torch.int32, device='cuda')
+    rnd = [torch.as_tensor(np.ascontiguousarray(x)).cuda() for x in (sites, moves, us)]
+    _lib.call('fk_mh_rbm', *[_lib.ptr(t) for t in m.parts()], n, m.n_hidden, *shape, kind, C, n_burn, spc, unused,
+              _lib.ptr(state), _lib.ptr(out), _lib.ptr(accepts), _lib.ptr(logpsi), *[_lib.ptr(t) for t in rnd], 0,
+              _lib.ptr(flag), _lib.stream_ptr())
+    assert not flag.item()
+    return out, state, accepts, logpsi
+
+
+@pytest.mark.parametrize('kind', [0, 1])
+@pytest.mark.parametrize('shape,alpha,per_cu', [((3, 4), 6, (9,)), ((4, 4), 8, (9,)), ((3, 4), 17, (5, 9)),
+                                                ((4, 4), 16, (5, 9)), ((3, 4), 25, (3, 5)), ((4, 4), 32, (3, 5))])
+def test_mh_rbm_chains_of_many_hidden_units(rng, shape, alpha, per_cu, kind):
+    """72 to 512 hidden units, in a wave per 64 of them (9 chains) and, with
+    per_cu chains a CU, two or four units a lane; full and ragged last waves;
+    280 steps, past the 64 that are drawn at once and the refresh of theta at
+    256.  The 9 chains follow the oracle's rule up to a near tie, and in every
+    form they are the same bits.  The final log psi is kept by 24 steps of
+    updates of theta since the refresh (2^-24 of |theta| < 1 each, in up to 512
+    units): 1e-5 as log psi itself, and 2e-4 of its phase."""
+    gpu_banner(f'mh rbm kind={kind} {shape} alpha={alpha}')
+    m = _rbm(shape, alpha, 0.05, seed=11)
+    n, few, burn, spc, unused = shape[0] * shape[1], 9, 40, 3, 79
+    steps = burn + spc * (unused + 1)
+    cu = torch.cuda.get_device_properties(0).multi_processor_count
+    most = max(per_cu) * cu
+    sites = rng.integers(0, n, size=(steps, most)).astype(np.int32)
+    moves = rng.integers(0, 9, size=(steps, most)).astype(np.int32)
+    us = rng.random((steps, most))
+    start = torch.as_tensor(rng.choice([-1, 1], size=(most, n)).astype(np.int8)).cuda()
+    base = _mh_rbm(m, shape, kind, start[:few], sites[:, :few], moves[:, :few], us[:, :few], burn, spc, unused)
+    ref, _, first_tie = _oracle_chain(lambda x: _oracle_lp(m, x), start[:few].cpu().numpy().reshape((few,) + shape),
+                                      sites[:, :few], moves[:, :few], us[:, :few], kind, shape, burn, spc, unused)
+    clean = _check_divergence(base[0].cpu().numpy().reshape((few, spc) + shape), ref, first_tie, burn, unused)
+    assert clean > 0.5, clean
+    lp = m.log_psi(base[1].reshape((few,) + shape)).cpu().numpy().reshape(-1)
+    got = torch.view_as_complex(base[3]).cpu().numpy()
+    assert np.abs(got.real - lp.real).max() < 1e-5 * (np.abs(lp.real).max() + 1)
+    assert np.abs(np.angle(np.exp(1j * (got.imag - lp.imag)))).max() < 2e-4
+    for k in per_cu:
+        C = k * cu
+        many = _mh_rbm(m, shape, kind, start[:C], sites[:, :C], moves[:, :C], us[:, :C], burn, spc, unused)
+        for a, b in zip(base, many):
+            assert torch.equal(a, b[:few])
