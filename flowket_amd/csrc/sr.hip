@@ -139,18 +139,19 @@ __global__ __launch_bounds__(DOT_BLOCKS) void dot_totals_kernel(const double* __
 
 // u_b = sum_k (O_bk - Obar_k) v_k = O_b.v - Obar.v (complex).  A workgroup
 // covers ROWS rows (each v_k read once for them) of column chunk blockIdx.y;
-// Obar.v in FP64, from its partial dots ov, is subtracted at the end.  With P
+// Obar.v in FP64 is subtracted at the end: the totals ov[0], ov[1] for several
+// rows, the sums of its partial dots ov for one.  With P
 // a multiple of 4 the rows are streamed as float4.  With one chunk u is
 // written here, with more the chunk's FP64 sums go to part ([chunk][row][2])
-// for ov_finish_kernel.
+// for ov_finish_kernel.  LOADS: iterations whose loads are in flight together.
 constexpr int64_t OV_PARTS = 8192;  // (chunk, row) sums that the scratch holds
 
-template <int ROWS>
+template <int ROWS, int LOADS>
 __global__ __launch_bounds__(256) void o_times_v_kernel(const float* __restrict__ ore, const float* __restrict__ oim,
                                                         const double* __restrict__ ov, const float* __restrict__ v,
                                                         int64_t B, int64_t P, double* __restrict__ part,
                                                         float* __restrict__ u) {
-  __shared__ double red[256];
+  __shared__ double red[2 * ROWS][256];
   const int64_t b0 = (int64_t)blockIdx.x * ROWS;
   double dr[ROWS], di[ROWS];
   float ar[ROWS], ai[ROWS];
@@ -161,7 +162,7 @@ __global__ __launch_bounds__(256) void o_times_v_kernel(const float* __restrict_
     const int64_t P4 = P >> 2;
     const int64_t k1 = P4 * (blockIdx.y + 1) / gridDim.y;
     const f32x4* v4 = reinterpret_cast<const f32x4*>(v);
-#pragma unroll 4
+#pragma unroll LOADS
     for (int64_t k = P4 * blockIdx.y / gridDim.y + threadIdx.x; k < k1; k += 256) {
       const f32x4 vk = v4[k];
 #pragma unroll
@@ -198,22 +199,35 @@ __global__ __launch_bounds__(256) void o_times_v_kernel(const float* __restrict_
     }
   }
   double ovr = 0.0, ovi = 0.0;
-  if (!part) {
-    ovr = dot_total(ov, red);
-    ovi = dot_total(ov + DOT_BLOCKS, red);
+  if (ROWS > 1) {  // many workgroups: the totals are made once for them
+    ovr = ov[0];
+    ovi = ov[1];
+  } else if (!part) {
+    ovr = dot_total(ov, red[0]);
+    ovi = dot_total(ov + DOT_BLOCKS, red[0]);
+    __syncthreads();
   }
 #pragma unroll
   for (int r = 0; r < ROWS; ++r) {
-    const double sr = block_sum(dr[r] + ar[r], red), si = block_sum(di[r] + ai[r], red);
-    if (threadIdx.x == 0 && b0 + r < B) {
-      if (part) {
-        part[((int64_t)blockIdx.y * B + b0 + r) * 2] = sr;
-        part[((int64_t)blockIdx.y * B + b0 + r) * 2 + 1] = si;
-      } else {
-        u[2 * (b0 + r)] = (float)(sr - ovr);
-        u[2 * (b0 + r) + 1] = (float)(si - ovi);
-      }
+    red[2 * r][threadIdx.x] = dr[r] + ar[r];
+    red[2 * r + 1][threadIdx.x] = di[r] + ai[r];
+  }
+  __syncthreads();
+  for (int st = 128; st > 0; st >>= 1) {
+    if ((int)threadIdx.x < st) {
+#pragma unroll
+      for (int r = 0; r < 2 * ROWS; ++r) red[r][threadIdx.x] += red[r][threadIdx.x + st];
     }
+    __syncthreads();
+  }
+  const int r = threadIdx.x;
+  if (r >= ROWS || b0 + r >= B) return;
+  if (part) {
+    part[((int64_t)blockIdx.y * B + b0 + r) * 2] = red[2 * r][0];
+    part[((int64_t)blockIdx.y * B + b0 + r) * 2 + 1] = red[2 * r + 1][0];
+  } else {
+    u[2 * (b0 + r)] = (float)(red[2 * r][0] - ovr);
+    u[2 * (b0 + r) + 1] = (float)(red[2 * r + 1][0] - ovi);
   }
 }
 
@@ -267,38 +281,77 @@ __global__ void center_pairs_kernel(float* __restrict__ u, int64_t B, const doub
 
 // out_k = scale * Re[sum_b conj(O_bk - Obar_k) u_b] + shift * v_k, columns in
 // fours (a column kernel, see o_mean4_kernel); FP32 over 64 rows, then FP64.
-__global__ __launch_bounds__(64 * COL_WAVES) void oh_times_u4_kernel(
-    const f32x4* __restrict__ ore, const f32x4* __restrict__ oim, const float* __restrict__ mre,
-    const float* __restrict__ mim, const float* __restrict__ u, const double* __restrict__ usum, int64_t B, int64_t P4,
-    double scale, double shift, const float* __restrict__ v, float* __restrict__ out) {
+struct OhArgs {
+  const f32x4 *ore, *oim;
+  const float *mre, *mim, *u;
+  const double* usum;
+  int64_t B, P4;
+  double scale, shift;
+  const float* v;
+  float* out;
+};
+
+// the sums of columns t of rows [b0, b1)
+__device__ __forceinline__ void oh_rows(const OhArgs& a, int64_t t, int64_t b0, int64_t b1, double (&acc)[4]) {
+  for (int64_t c0 = b0; c0 < b1; c0 += 64) {
+    const int64_t c1 = c0 + 64 < b1 ? c0 + 64 : b1;
+    f32x4 part = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 8
+    for (int64_t b = c0; b < c1; ++b)
+      part += a.ore[b * a.P4 + t] * a.u[2 * b] + a.oim[b * a.P4 + t] * a.u[2 * b + 1];
+#pragma unroll
+    for (int c = 0; c < 4; ++c) acc[c] += part[c];
+  }
+}
+__device__ __forceinline__ void oh_store(const OhArgs& a, int64_t k, double r) {
+  r = a.scale * (r - ((double)a.mre[k] * a.usum[0] + (double)a.mim[k] * a.usum[1]));
+  if (a.v) r += a.shift * (double)a.v[k];
+  a.out[k] = (float)r;
+}
+
+__global__ __launch_bounds__(64 * COL_WAVES) void oh_times_u4_kernel(OhArgs a) {
   extern __shared__ double red[];  // [waves][4][64]
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), nw = blockDim.x >> 6;
   const int64_t t = (int64_t)blockIdx.x * 64 + lane;
   int64_t b0, b1;
-  wave_rows(B, w, nw, b0, b1);
+  wave_rows(a.B, w, nw, b0, b1);
   double acc[4] = {0.0, 0.0, 0.0, 0.0};
-  if (t < P4) {
-    for (int64_t c0 = b0; c0 < b1; c0 += 64) {
-      const int64_t c1 = c0 + 64 < b1 ? c0 + 64 : b1;
-      f32x4 part = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll 8
-      for (int64_t b = c0; b < c1; ++b) part += ore[b * P4 + t] * u[2 * b] + oim[b * P4 + t] * u[2 * b + 1];
-#pragma unroll
-      for (int c = 0; c < 4; ++c) acc[c] += part[c];
-    }
-  }
+  if (t < a.P4) oh_rows(a, t, b0, b1, acc);
 #pragma unroll
   for (int c = 0; c < 4; ++c) red[(w * 4 + c) * 64 + lane] = acc[c];
   __syncthreads();
-  if (w > 0 || t >= P4) return;
+  if (w > 0 || t >= a.P4) return;
 #pragma unroll
   for (int c = 0; c < 4; ++c) {
     double r = 0.0;
     for (int q = 0; q < nw; ++q) r += red[(q * 4 + c) * 64 + lane];
-    const int64_t k = 4 * t + c;
-    r = scale * (r - ((double)mre[k] * usum[0] + (double)mim[k] * usum[1]));
-    if (v) r += shift * (double)v[k];
-    out[k] = (float)r;
+    oh_store(a, 4 * t + c, r);
+  }
+}
+
+// The same for columns that (almost) fill the chip by themselves: CG waves of
+// columns and NW ranges of rows a workgroup, registers for eight waves per SIMD.
+template <int CG, int NW>
+__global__ __launch_bounds__(64 * CG * NW, 8) void oh_times_u4_wide_kernel(OhArgs a) {
+  __shared__ double red[NW][4][64 * CG];
+  const int c = threadIdx.x % (64 * CG), w = __builtin_amdgcn_readfirstlane(threadIdx.x / (64 * CG));
+  const int64_t t = (int64_t)blockIdx.x * (64 * CG) + c;
+  int64_t b0, b1;
+  wave_rows(a.B, w, NW, b0, b1);
+  double acc[4] = {0.0, 0.0, 0.0, 0.0};
+  if (t < a.P4) oh_rows(a, t, b0, b1, acc);
+  if constexpr (NW > 1) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) red[w][e][c] = acc[e];
+    __syncthreads();
+  }
+  if (w > 0 || t >= a.P4) return;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    double r = acc[e];
+#pragma unroll
+    for (int q = 1; q < NW; ++q) r += red[q][e][c];
+    oh_store(a, 4 * t + e, r);
   }
 }
 
@@ -638,7 +691,10 @@ int fk_o_times_v(const float* o_re, const float* o_im, const float* mean_re, con
   // Four rows a workgroup where that still gives every CU four workgroups;
   // else one row, and where even the rows are too few, column chunks of at
   // least 8 KB (1024 rows of 215,492 columns: 788 us in groups of four rows,
-  // four waves per CU; 299 us, 5.9 TB/s, one row each).
+  // four waves per CU; 299 us, 5.9 TB/s, one row each).  Four workgroups a CU need
+  // the loads of four iterations in flight (4096 rows x 849,156: 4.98 ms without,
+  // 4.74 with), six and more are faster without (8192 rows: 9.24 and 9.78: eight a
+  // CU, of which the registers of four loads leave seven, so a second round).
   const int64_t want = 4LL * device_cu_count();
   const int64_t rows = batch >= 4 * want ? 4 : 1;
   int64_t chunks = 1;
@@ -649,12 +705,16 @@ int fk_o_times_v(const float* o_re, const float* o_im, const float* mean_re, con
     if (chunks < 1) chunks = 1;
   }
   double* part = chunks > 1 ? scratch + 2 * DOT_BLOCKS : nullptr;
-  if (rows == 4)
-    hipLaunchKernelGGL(o_times_v_kernel<4>, dim3(div_up(batch, 4)), dim3(256), 0, s, o_re, o_im, scratch, v, batch,
-                       n_params, part, u);
-  else
-    hipLaunchKernelGGL(o_times_v_kernel<1>, dim3((unsigned)batch, (unsigned)chunks), dim3(256), 0, s, o_re, o_im,
+  if (rows == 4) {
+    double* totals = scratch + 2 * DOT_BLOCKS;
+    hipLaunchKernelGGL(dot_totals_kernel, dim3(2), dim3(DOT_BLOCKS), 0, s, scratch, totals);
+    FK_CHECK_LAUNCH();
+    hipLaunchKernelGGL((batch > 5 * want ? o_times_v_kernel<4, 1> : o_times_v_kernel<4, 4>), dim3(div_up(batch, 4)),
+                       dim3(256), 0, s, o_re, o_im, totals, v, batch, n_params, part, u);
+  } else {
+    hipLaunchKernelGGL((o_times_v_kernel<1, 4>), dim3((unsigned)batch, (unsigned)chunks), dim3(256), 0, s, o_re, o_im,
                        scratch, v, batch, n_params, part, u);
+  }
   FK_CHECK_LAUNCH();
   if (part) {
     hipLaunchKernelGGL(ov_finish_kernel, dim3(div_up(batch, 256)), dim3(256), 0, s, part, chunks, scratch, batch, u);
@@ -676,10 +736,26 @@ int fk_oh_times_u(const float* o_re, const float* o_im, const float* mean_re, co
                        scratch2, batch, n_params, scale, shift, v, out);
   } else {
     const int64_t p4 = n_params / 4;
-    const int nw = col_waves(div_up(p4, 64), batch);
-    hipLaunchKernelGGL(oh_times_u4_kernel, dim3(div_up(p4, 64)), dim3(64 * nw), (size_t)nw * 4 * 64 * sizeof(double), s,
-                       reinterpret_cast<const f32x4*>(o_re), reinterpret_cast<const f32x4*>(o_im), mean_re, mean_im, u,
-                       scratch2, batch, p4, scale, shift, v, out);
+    const OhArgs a{reinterpret_cast<const f32x4*>(o_re), reinterpret_cast<const f32x4*>(o_im), mean_re, mean_im, u,
+                   scratch2, batch, p4, scale, shift, v, out};
+    // By waves of columns per CU: from 10 on they need no second range of rows,
+    // from 7 on two ranges do, with registers for eight waves per SIMD; fewer are
+    // dealt as in o_mean.  (A thread per four columns over all rows / dealt as in
+    // o_mean / this, ms: 8192 rows x 849,156 9.59 / 10.03 / 9.47, x 700,000 7.63 /
+    // 7.97 / 7.74, 2048 x 524,284 1.52 / 1.70 / 1.47; 1024 x 849,156 1.24 / 1.34 /
+    // 1.17; 4096 x 430,000 2.71 / 2.41 dealt.)
+    const int64_t per_cu = p4 / (64LL * device_cu_count());
+    if (per_cu >= 12) {
+      hipLaunchKernelGGL((oh_times_u4_wide_kernel<2, 1>), dim3(div_up(p4, 128)), dim3(128), 0, s, a);
+    } else if (per_cu >= 10) {
+      hipLaunchKernelGGL((oh_times_u4_wide_kernel<1, 1>), dim3(div_up(p4, 64)), dim3(64), 0, s, a);
+    } else if (per_cu >= 7) {
+      hipLaunchKernelGGL((oh_times_u4_wide_kernel<2, 2>), dim3(div_up(p4, 128)), dim3(256), 0, s, a);
+    } else {
+      const int nw = col_waves(div_up(p4, 64), batch);
+      hipLaunchKernelGGL(oh_times_u4_kernel, dim3(div_up(p4, 64)), dim3(64 * nw), (size_t)nw * 4 * 64 * sizeof(double),
+                         s, a);
+    }
   }
   FK_CHECK_LAUNCH();
   return FK_OK;

@@ -423,3 +423,12 @@ def test_sr_products_row_and_chunk_splits(B, P):
     refh = 0.5 * (oc.conj().T @ torch.view_as_complex(w.double())).real + 2.0 * v.double()
     scale = 0.5 * (o.abs() ** 2).sum(dim=0).sqrt() * w.abs().max().double() + 2.0 * v.abs().double()
     assert ((out.double() - refh).abs() / scale).max().item() < 1e-6
+
+
+@pytest.mark.parametrize('B,P', [(5, 458748), (130, 458752), (3, 655356), (129, 655364), (66, 786428), (67, 786436),
+                                 (1, 786432), (5120, 260), (5123, 260), (5124, 1028)])
+def test_sr_products_wide_rows_and_many_rows(B, P):
+    """The same where the columns fill the chip (7, 10 and 12 waves of them per
+    CU, a column group more or less) and, for many rows, on both sides of the
+    rule for loads in flight."""
+    test_sr_products_row_and_chunk_splits(B, P)
