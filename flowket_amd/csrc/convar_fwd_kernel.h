@@ -465,9 +465,13 @@ __global__ __launch_bounds__(64 * NWAVE) void convar_fwd_kernel(FwdArgs a) {
   };
   int64_t m0, M = 0;
   // (not in FP32, where 512 10x10 C 32 depth 20 configurations took 1.11 ms with
-  // a.T and 1.14 to 1.16 with a tile computed here)
-  if constexpr (PREC != FK_PREC_FP32) M = count(m0);
-  const int T = PREC == FK_PREC_FP32 ? a.T : __builtin_amdgcn_readfirstlane(fwd_tile(a.T, M, gridDim.x));
+  // a.T and 1.14 to 1.16 with a tile computed here, nor in HG, whose largest
+  // tile is one configuration: there it only takes scalar registers, and the row
+  // reuse of 20x20 C 64 bf16, 64 samples, runs two of its ranges in 8.1 ms for
+  // 6.4)
+  constexpr bool DEV_TILE = PREC != FK_PREC_FP32 && !HG;
+  if constexpr (DEV_TILE) M = count(m0);
+  const int T = DEV_TILE ? __builtin_amdgcn_readfirstlane(fwd_tile(a.T, M, gridDim.x)) : a.T;
   // NPX = T*HW real pixels, covered by 16-pixel tiles.
   // Each buffer holds the NPX pixels plus ZERO_PIX all-zero pixels that padding
   // taps and the tile lanes past NPX read: a lane whose tap target q falls
@@ -509,7 +513,7 @@ __global__ __launch_bounds__(64 * NWAVE) void convar_fwd_kernel(FwdArgs a) {
   const int H = a.H, W = a.W, HW = a.HW;
   const int HR = ROWS ? a.HR : H, ROW0 = ROWS ? a.ROW0 : 0;
   const int gofs = ROWS ? (a.R0 - ROW0) * W : 0;  // global index of a configuration's LDS pixel 0
-  const int ntiles = (PREC == FK_PREC_FP32 ? a.npix : T * HWC + 15) >> 4;
+  const int ntiles = (DEV_TILE ? T * HWC + 15 : a.npix) >> 4;
   const int nt = (ntiles > wave) ? (ntiles - wave + NW - 1) / NW : 0;
 
   int pix[MAXT], pi[MAXT], pj[MAXT];
@@ -561,7 +565,7 @@ __global__ __launch_bounds__(64 * NWAVE) void convar_fwd_kernel(FwdArgs a) {
     reinterpret_cast<uint32_t*>(H1 + NPX * PIXB)[z] = 0u;
   }
 
-  if constexpr (PREC == FK_PREC_FP32) M = count(m0);
+  if constexpr (!DEV_TILE) M = count(m0);
   const int64_t ngroups = (M + T - 1) / T;
   const int nb = a.nblocks;
   const frag* wall = reinterpret_cast<const frag*>(a.w);
