@@ -62,6 +62,7 @@ SIGNATURES = {
     'fk_convar_get_schedule': (_I32, [_I32, _I32, _I32, _I32, _I32, _I32]),
     'fk_ar_draw_site': (ctypes.c_int, [_P, _P, _I64, _I32, _I32, _P, _P]),
     'fk_fast_sampler_workspace_bytes': (_I64, [_I32, _I32, _I32, _I32, _I32, _I64]),
+    'fk_fast_sampler_waves': (_I32, [_I32, _I32, _I32, _I32, _I32, _I64]),
     'fk_fast_sample': (ctypes.c_int, [_P, _P, _I32, _I32, _I32, _I32, _I32, _I32, _I64, _P, _P, _P, _P, _P]),
     'fk_convar_grad_workspace_bytes': (_I64, [_I32, _I32, _I32, _I32, _I64]),
     'fk_convar_grad': (ctypes.c_int, [_P, _I32, _I32, _I32, _I32, _I32, _P, _I64, _P, _P, _P, _I64, _P, _P]),

@@ -158,10 +158,12 @@ constexpr int fast_lb() {
 // .. + 3 stay inside the C or C/2 biases of the M-tiles that read them).
 __device__ __forceinline__ f32x4 ldq4(const float* p) { return *reinterpret_cast<const f32x4*>(p); }
 
-// The workgroup-per-tile kernel: the cache bytes of a tile, whether it takes a
-// network (channels: the kernel width), and its launch.
+// The workgroup-per-tile kernel: the cache bytes of a tile, whether it can take
+// a network (channels: the kernel width), whether it takes a batch of it, and
+// its launch.
 int64_t fast_mw_tile_bytes(int H, int W, int nb, int channels, int precision);
 bool fast_mw_supported(int H, int W, int nb, int channels, int precision);
+bool fast_mw_takes(int H, int W, int nb, int channels, int precision, int64_t tiles);
 int launch_fast_mw(const SampArgs& a, int channels, int precision, int act, int64_t tiles, hipStream_t s);
 
 }  // namespace fk

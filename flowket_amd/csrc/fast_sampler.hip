@@ -17,10 +17,11 @@
 // accumulation order and the roundings are those of the fused forward kernel,
 // so the draws equal the plain sampler's draws given the same uniforms.
 //
-// Most networks take the workgroup-per-tile kernel of fast_sampler_mw.hip;
-// this one draws from those that it does not take (fast_mw_supported).  Its
-// whole-row form stays for two-block networks on rows of at most VROW_MAX
-// pixels (10x10, 1024 samples: 0.32 ms against 0.48 without it).
+// Most calls take the workgroup-per-tile kernel of fast_sampler_mw.hip; this
+// one draws where that cannot or is slower (fast_mw_takes: two-block networks,
+// narrow rows and shallow networks in batches that fill the chip).  Its
+// whole-row form is for 16-bit 32-channel networks on rows of at most VROW_MAX
+// pixels (two blocks, 10x10, 1024 samples: 0.32 ms against 0.48 without it).
 #include "fast_sampler.h"
 
 #include <type_traits>
@@ -1030,14 +1031,21 @@ static bool fast_whole_row(int W, int channels, int precision) {
 // Per-tile cache: (3 nb - 2) activation buffers of HW + 2 pixels, the spins
 // and, for the whole-row kernel, one row of concatenation partial sums per
 // block (FP32, MT quads per lane, VROW_MAX columns).
-int64_t fast_tile_bytes(int H, int W, int nb, int channels, int precision) {
-  if (fast_mw_supported(H, W, nb, channels, precision)) return fast_mw_tile_bytes(H, W, nb, channels, precision);
+static int64_t fast_one_wave_tile_bytes(int H, int W, int nb, int channels, int precision) {
   const int esz = precision == FK_PREC_FP32 ? 4 : 2;
   const int64_t pb = 16LL * channels * esz;
   const int64_t HW = (int64_t)H * W;
   int64_t b = (int64_t)(3 * nb - 2) * (HW + 2) * pb + HW * 16 * 4;
   if (fast_whole_row(W, channels, precision)) b += (int64_t)nb * VROW_MAX * 64 * (channels / 16) * 16;
   return b;
+}
+// the workspace of a tile: that of either kernel, since a smaller batch in the
+// same workspace may take the other one
+static int64_t fast_tile_bytes(int H, int W, int nb, int channels, int precision) {
+  const int64_t one = fast_one_wave_tile_bytes(H, W, nb, channels, precision);
+  if (!fast_mw_supported(H, W, nb, channels, precision)) return one;
+  const int64_t mw = fast_mw_tile_bytes(H, W, nb, channels, precision);
+  return mw > one ? mw : one;
 }
 
 template <int PREC, int C, bool WR>
@@ -1078,6 +1086,14 @@ int64_t fk_fast_sampler_workspace_bytes(int32_t H, int32_t W, int32_t depth, int
   return tiles * fast_tile_bytes(H, W, num_causal_blocks(depth), fast_channels(channels, precision), precision);
 }
 
+int32_t fk_fast_sampler_waves(int32_t H, int32_t W, int32_t depth, int32_t channels, int32_t precision,
+                              int64_t batch) {
+  if (H < 1 || W < 1 || depth < 1 || batch < 0 || !fast_sampler_supported(channels, precision)) return -1;
+  return fast_mw_takes(H, W, num_causal_blocks(depth), fast_channels(channels, precision), precision, (batch + 15) / 16)
+             ? 4
+             : 1;
+}
+
 int fk_fast_sample(const void* wpacked, const float* aux, int32_t precision, int32_t H, int32_t W, int32_t depth,
                    int32_t channels, int32_t activation, int64_t batch, const double* uniforms, void* workspace,
                    int8_t* out, float* cond_logp, void* stream) {
@@ -1103,11 +1119,14 @@ int fk_fast_sample(const void* wpacked, const float* aux, int32_t precision, int
   a.cond = cond_logp;
   a.cache = reinterpret_cast<uint8_t*>(workspace);
   const int CP = fast_channels(channels, precision);
-  a.tile_bytes = fast_tile_bytes(H, W, a.nb, CP, precision);
   const int64_t tiles = (batch + 15) / 16;
   FK_REQUIRE(tiles <= 0x7fffffff, "fk_fast_sample: batch too large");
   hipStream_t s = (hipStream_t)stream;
-  if (fast_mw_supported(H, W, a.nb, CP, precision)) return launch_fast_mw(a, CP, precision, activation, tiles, s);
+  if (fast_mw_takes(H, W, a.nb, CP, precision, tiles)) {
+    a.tile_bytes = fast_mw_tile_bytes(H, W, a.nb, CP, precision);
+    return launch_fast_mw(a, CP, precision, activation, tiles, s);
+  }
+  a.tile_bytes = fast_one_wave_tile_bytes(H, W, a.nb, CP, precision);
   if (precision == FK_PREC_BF16) {
     if (CP == 32) return launch_fast<FK_PREC_BF16, 32>(a, activation, tiles, s);
     return launch_fast<FK_PREC_BF16, 64>(a, activation, tiles, s);

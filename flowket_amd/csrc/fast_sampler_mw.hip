@@ -823,14 +823,60 @@ int64_t fast_mw_tile_bytes(int H, int W, int nb, int channels, int precision) {
   return ((int64_t)(3 * nb - 2) * ((int64_t)H * W + 2) + mw_pad(W)) * pb + (int64_t)nb * W * channels * 64;
 }
 
-bool fast_mw_supported(int H, int W, int nb, int channels, int precision) {
+// Steps per super-tick of a network that the kernel can take, or 0.
+static int mw_steps_of(int H, int W, int nb, int channels, int precision) {
   // (the cache of a tile is addressed by 32-bit offsets)
-  if (fast_mw_tile_bytes(H, W, nb, channels, precision) >= 0x7fffffff) return false;
-  if (precision == FK_PREC_FP32 && channels == 64) return false;  // (its fragments are single floats: spills)
-  const int G = precision == FK_PREC_FP32   ? mw_steps_c<FK_PREC_FP32>(W, nb, channels)
-                : precision == FK_PREC_BF16 ? mw_steps_c<FK_PREC_BF16>(W, nb, channels)
-                                            : mw_steps_c<FK_PREC_FP16>(W, nb, channels);
-  return G > 0;
+  if (fast_mw_tile_bytes(H, W, nb, channels, precision) >= 0x7fffffff) return 0;
+  if (precision == FK_PREC_FP32 && channels == 64) return 0;  // (its fragments are single floats: spills)
+  return precision == FK_PREC_FP32   ? mw_steps_c<FK_PREC_FP32>(W, nb, channels)
+         : precision == FK_PREC_BF16 ? mw_steps_c<FK_PREC_BF16>(W, nb, channels)
+                                     : mw_steps_c<FK_PREC_FP16>(W, nb, channels);
+}
+
+bool fast_mw_supported(int H, int W, int nb, int channels, int precision) {
+  return mw_steps_of(H, W, nb, channels, precision) > 0;
+}
+
+// Rounds of workgroups over the chip (one per CU) up to which this kernel is
+// the faster one at 16-bit 64 channels and FP32.  Its waves share a tile, so it
+// needs rows that they can divide and blocks for its helpers (steps: helpers
+// that run; one of three for networks of four and six blocks); the one-wave
+// kernel runs several tiles a CU instead, as soon as there are as many.  Time of
+// this kernel over the other's, six rows, by rounds 1 / 2 / 4 / 8, depth 3 (one
+// step) and depth 5 (two):
+//   64 channels, W = 1   1.57 / 2.4 / 4.0 / 5.7    1.36 / 1.8 / 3.4 / 4.0
+//                W = 3   0.66 / 0.86 / 1.6 / 2.0   0.45 / 0.66 / 0.96 / 1.3
+//                W = 5   -    / 0.64 / 1.1 / 1.3   -    / 0.45 / 0.71 / 0.93
+//                W = 10  -    / 0.49 / 0.81 / 1.0  -    / 0.36 / 0.61 / 0.72
+//   FP32, 32     W = 1   2.0 / 3.4 / 5.4 / 7.8     1.9 / 2.7 / 5.2 / 6.1
+//                W = 3   0.73 / 1.1 / 2.1 / 2.4    0.57 / 0.86 / 1.4 / 1.7
+//                W = 5   -    / 0.86 / 1.4 / 1.7   -    / 0.60 / 0.98 / 1.2
+//                W = 10  -    / 0.68 / 1.1 / 1.3   -    / 0.45 / 0.74 / 0.88
+// (A single row has no vertical stack to divide; two rows have little of it.)
+static int mw_rounds(int H, int W, int steps, int precision) {
+  constexpr int ANY = 0x7fffffff;
+  if (H == 1) W = 7;
+  if (precision == FK_PREC_FP32) {
+    if (steps == 1) return W <= 2 ? 0 : W == 3 ? 1 : W < 8 ? 2 : 3;
+    return W < 5 ? W - 1 : W < 7 ? 4 : ANY;
+  }
+  if (steps == 1) return W <= 2 ? W - 1 : W < 5 ? 2 : W == 5 || H < 3 ? 3 : W < 10 || H < 6 ? 4 : ANY;
+  return W <= 2 ? 2 * (W - 1) : W < 5 ? 4 : ANY;
+}
+
+bool fast_mw_takes(int H, int W, int nb, int channels, int precision, int64_t tiles) {
+  const int steps = mw_steps_of(H, W, nb, channels, precision);
+  if (steps == 0) return false;
+  const int64_t cu = device_cu_count();
+  // 16-bit 32 channels (two workgroups a CU): all but four-block networks on
+  // narrow or two rows, which one wave draws faster once there is a second round,
+  // or a third (4x4, 6x6, 8x8, 32768 samples: 544 against 449 us, 1101 and 992,
+  // 1937 and 1838; 8x8, 16384: 977 and 1145; not 3x3, 282 and 315)
+  if (precision != FK_PREC_FP32 && channels == 32) {
+    const bool narrow = W <= 6 || H == 2;
+    return !(nb == 4 && H > 1 && H * W >= 12 && (narrow || W <= 8) && tiles > (narrow ? 2 : 4) * cu);
+  }
+  return (tiles + cu - 1) / cu <= mw_rounds(H, W, steps, precision);
 }
 
 template <int PREC, int C>

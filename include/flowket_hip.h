@@ -310,6 +310,11 @@ int fk_ar_draw_site(const float* cond_logp, const double* uniforms,
 int64_t fk_fast_sampler_workspace_bytes(int32_t H, int32_t W, int32_t depth,
                                         int32_t channels, int32_t precision,
                                         int64_t batch);
+/* Waves that draw 16 samples of such a batch: 4 (a workgroup) or 1; -1 where
+ * the sampler does not take the network.  The draws do not depend on it. */
+int32_t fk_fast_sampler_waves(int32_t H, int32_t W, int32_t depth,
+                              int32_t channels, int32_t precision,
+                              int64_t batch);
 int fk_fast_sample(const void* wpacked, const float* aux, int32_t precision,
                    int32_t H, int32_t W, int32_t depth, int32_t channels,
                    int32_t activation, int64_t batch, const double* uniforms,

@@ -89,3 +89,46 @@ def test_workgroup_per_tile_equals_plain(rng, shape, depth, C, act, prec, B):
     and precision.  Draws and conditionals are those of the plain sampler, bit
     for bit."""
     test_fast_equals_plain_given_uniforms(rng, shape, depth, C, act, prec, B)
+
+
+def _waves(shape, depth, C, prec, B):
+    from flowket_amd import _lib
+    code = {'fp32': _lib.FK_PREC_FP32, 'bf16': _lib.FK_PREC_BF16, 'fp16': _lib.FK_PREC_FP16}[prec]
+    return _lib.load().fk_fast_sampler_waves(*shape, depth, C, code, B)
+
+
+@pytest.mark.parametrize('shape,depth,C,act,prec,B,per_tile', [
+    # three steps per super-tick, four times as many blocks or a few more (operands four steps old), each width
+    ((4, 5), 7, 32, 'relu', 'fp16', 18, 4), ((3, 6), 8, 20, 'elu', 'bf16', 16, 4), ((4, 5), 7, 64, 'elu', 'bf16', 17, 4),
+    ((3, 6), 8, 48, 'relu', 'fp16', 20, 4), ((4, 5), 7, 32, 'elu', 'fp32', 16, 4), ((3, 6), 8, 24, 'relu', 'fp32', 19, 4),
+    # the widest rows that the LDS holds, and one pixel more
+    ((3, 63), 7, 32, 'relu', 'fp16', 20, 4), ((3, 64), 9, 32, 'elu', 'bf16', 20, 1), ((3, 34), 7, 64, 'relu', 'bf16', 17, 4),
+    ((3, 35), 7, 64, 'relu', 'bf16', 17, 1), ((3, 34), 8, 32, 'elu', 'fp32', 18, 4), ((2, 35), 8, 32, 'elu', 'fp32', 18, 1),
+    # rows of one pixel and of a few, where one wave is faster, and FP32 at 64 channels
+    ((5, 1), 5, 64, 'elu', 'fp16', 20, 1), ((4, 1), 8, 32, 'relu', 'fp32', 18, 1), ((4, 2), 3, 20, 'elu', 'fp32', 16, 1),
+    ((3, 2), 3, 40, 'relu', 'bf16', 16, 4), ((3, 4), 4, 64, 'elu', 'fp32', 17, 1)])
+def test_kernel_by_network_equals_plain(rng, shape, depth, C, act, prec, B, per_tile):
+    """The draws of either kernel are those of the plain sampler, bit for bit;
+    per_tile waves draw 16 of them."""
+    assert _waves(shape, depth, C, prec, B) == per_tile
+    test_fast_equals_plain_given_uniforms(rng, shape, depth, C, act, prec, B)
+
+
+@pytest.mark.parametrize('shape,depth,C,act,prec,rounds', [
+    ((4, 4), 3, 32, 'relu', 'fp16', 2), ((3, 6), 3, 24, 'elu', 'bf16', 2), ((3, 3), 3, 64, 'relu', 'bf16', 2),
+    ((2, 2), 5, 48, 'elu', 'fp16', 2), ((3, 8), 3, 32, 'relu', 'fp16', 4), ((2, 3), 5, 32, 'elu', 'fp32', 2), ((3, 5), 3, 32, 'relu', 'fp32', 2)])
+def test_kernel_by_batch_equals_plain(rng, shape, depth, C, act, prec, rounds):
+    """A batch of as many tiles as workgroups in ``rounds`` rounds over the chip
+    is drawn by four waves a tile and a larger one by one wave, in the same
+    workspace (chunks of the larger batch, and the rest of it)."""
+    import flowket_amd as fk
+    cu = torch.cuda.get_device_properties(0).multi_processor_count
+    B = rounds * cu * 16
+    assert _waves(shape, depth, C, prec, B) == 4 and _waves(shape, depth, C, prec, B + 1) == 1
+    m = _machine(shape, depth, C, act, prec)
+    total = B + 17 + 40
+    u = rng.random((total,) + shape)
+    plain = next(fk.AutoregressiveSampler(m, total, uniforms=u))
+    assert torch.equal(next(fk.FastAutoregressiveSampler(m, total, uniforms=u)), plain)
+    assert torch.equal(next(fk.FastAutoregressiveSampler(m, total, mini_batch_size=B + 17, uniforms=u)), plain)
+    assert torch.equal(next(fk.FastAutoregressiveSampler(m, B, uniforms=u[:B])), plain[:B])
