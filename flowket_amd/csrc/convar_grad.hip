@@ -1079,16 +1079,17 @@ int launch_plan(K kern, const GradPlan& p, hipStream_t s, const BwdArgs& a) {
   return FK_OK;
 }
 
+// threads of a workgroup that has a CU to itself, tensors in LDS (grad_plan)
+constexpr int resident_threads(int C, int mode) { return C == 32 && mode != GRAD_JVP ? 1024 : 512; }
+
 template <int C, int ACT, int MODE>
 int launch_mode(const GradPlan& p, const BwdArgs& a, hipStream_t s) {
   if (!p.resident) return launch_plan(convar_grad_kernel3<C, ACT, MODE, false, 512>, p, s, a);
-  if constexpr (C == 32 && MODE != GRAD_JVP)
-    if (p.threads == 1024) return launch_plan(convar_grad_kernel3<C, ACT, MODE, true, 1024>, p, s, a);
   if constexpr (MODE != GRAD_VJP) {
     if (p.threads == 128) return launch_plan(convar_grad_kernel3<C, ACT, MODE, true, 128>, p, s, a);
     if (p.threads == 256) return launch_plan(convar_grad_kernel3<C, ACT, MODE, true, 256>, p, s, a);
   }
-  return launch_plan(convar_grad_kernel3<C, ACT, MODE, true, 512>, p, s, a);
+  return launch_plan(convar_grad_kernel3<C, ACT, MODE, true, resident_threads(C, MODE)>, p, s, a);
 }
 template <int C, int ACT>
 int launch_act(const GradPlan& p, const BwdArgs& a, int mode, hipStream_t s) {
@@ -1121,7 +1122,7 @@ GradPlan grad_plan(const BwdArgs& a, int mode) {
   // against 512 (two): 10x10 C 32, 2048 samples, VJP 15.6 and 16.6, O 24.7 and
   // 26.6, JVP 11.4 both; C 64 has no registers for 1024 (10x10, 1024 samples,
   // VJP 14.4 and 13.0).
-  p.threads = p.resident && C == 32 && mode != GRAD_JVP ? 1024 : 512;
+  p.threads = p.resident ? resident_threads(C, mode) : 512;
   p.per_cu = 1;
   if (p.resident && mode != GRAD_VJP) {
     if (4 * p.lds <= 156 * 1024 && batch > 2 * cu) {

@@ -815,7 +815,11 @@ static int mw_steps(int W, int nb) {
 
 template <int PREC>
 static int mw_steps_c(int W, int nb, int channels) {
-  return channels == 32 ? mw_steps<PREC, 32>(W, nb) : channels == 64 ? mw_steps<PREC, 64>(W, nb) : 0;
+  if (channels == 32) return mw_steps<PREC, 32>(W, nb);
+  // (FP32 at 64 channels: its fragments are single floats, which spill)
+  if constexpr (PREC != FK_PREC_FP32)
+    if (channels == 64) return mw_steps<PREC, 64>(W, nb);
+  return 0;
 }
 
 int64_t fast_mw_tile_bytes(int H, int W, int nb, int channels, int precision) {
@@ -827,7 +831,6 @@ int64_t fast_mw_tile_bytes(int H, int W, int nb, int channels, int precision) {
 static int mw_steps_of(int H, int W, int nb, int channels, int precision) {
   // (the cache of a tile is addressed by 32-bit offsets)
   if (fast_mw_tile_bytes(H, W, nb, channels, precision) >= 0x7fffffff) return 0;
-  if (precision == FK_PREC_FP32 && channels == 64) return 0;  // (its fragments are single floats: spills)
   return precision == FK_PREC_FP32   ? mw_steps_c<FK_PREC_FP32>(W, nb, channels)
          : precision == FK_PREC_BF16 ? mw_steps_c<FK_PREC_BF16>(W, nb, channels)
                                      : mw_steps_c<FK_PREC_FP16>(W, nb, channels);
@@ -895,7 +898,7 @@ int launch_fast_mw(const SampArgs& a, int channels, int precision, int act, int6
     return channels == 32 ? launch_mw<FK_PREC_BF16, 32>(a, act, tiles, s) : launch_mw<FK_PREC_BF16, 64>(a, act, tiles, s);
   if (precision == FK_PREC_FP16)
     return channels == 32 ? launch_mw<FK_PREC_FP16, 32>(a, act, tiles, s) : launch_mw<FK_PREC_FP16, 64>(a, act, tiles, s);
-  return channels == 32 ? launch_mw<FK_PREC_FP32, 32>(a, act, tiles, s) : launch_mw<FK_PREC_FP32, 64>(a, act, tiles, s);
+  return launch_mw<FK_PREC_FP32, 32>(a, act, tiles, s);
 }
 
 }  // namespace fk

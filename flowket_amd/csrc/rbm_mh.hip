@@ -31,14 +31,6 @@ __device__ __forceinline__ float lncosh_re(float x, float y) {
   const float e2 = expf(-2.0f * ax);
   return ax - 0.69314718055994531f + 0.5f * log1pf(e2 * e2 + 2.0f * e2 * cosf(2.0f * y));
 }
-__device__ __forceinline__ float lncosh_im(float x, float y) {
-  // arg(e^{z-|x|} + e^{-z-|x|}) = atan2(Im, Re)
-  const float ax = fabsf(x);
-  const float e1 = expf(x - ax), e2 = expf(-x - ax);
-  float sy, cy;
-  sincosf(y, &sy, &cy);
-  return atan2f((e1 - e2) * sy, (e1 + e2) * cy);
-}
 
 // Sum over the wave, the butterfly v[l] + v[l ^ 32], then ^ 16, 8, 4, 2, 1, in
 // lane-permuting vector instructions: the halves and rows are exchanged by
@@ -63,8 +55,9 @@ __device__ __forceinline__ float wave_sum(float v) {
   return dpp_add<0xb1>(v);  // quad_perm [1, 0, 3, 2]
 }
 
-// lncosh(x + iy) with one exponential: of e^{x-|x|} and e^{-x-|x|} one is 1
-// and the other e^{-2|x|}, the e2 of lncosh_re.
+// Both parts, the imaginary one as the argument of e^{z-|x|} + e^{-z-|x|}, with
+// one exponential: of e^{x-|x|} and e^{-x-|x|} one is 1 and the other e^{-2|x|},
+// the e2 of lncosh_re.
 __device__ __forceinline__ void lncosh(float x, float y, float& re, float& im) {
   const float ax = fabsf(x);
   const float e = expf(-2.0f * ax);
