@@ -1109,6 +1109,13 @@ GradPlan grad_plan(const BwdArgs& a, int mode) {
        reinterpret_cast<uintptr_t>(a.tangent)) & 15)
     return p;
   const int64_t cu = device_cu_count();
+  // Lattices of one pixel tile at 64 channels: a sample is little but its weight
+  // gradients' way through the partial rows, for which four workgroups of the
+  // other kernel take turns better than one, once each has several samples (VJP,
+  // ms, this kernel and the other: 2x2 depth 3, 2048 samples 3.08 and 3.24, 4096
+  // 5.90 and 5.57, 16384 22.8 and 19.3; 4x4 depth 3, 4096 samples 6.06 and 6.24,
+  // 16384 23.5 and 22.3; two blocks, 3x3, 16384: 8.99 and 9.43).
+  if (mode == GRAD_VJP && C == 64 && HW <= 16 && a.nb > 2 && batch > (HW <= 6 ? 12 : 24) * cu) return p;
   const int tiles = mode == GRAD_JVP ? 8 : 5;
   p.resident = plan_lds(HW, C, tiles) <= 158 * 1024;
   p.lds = plan_lds(HW, C, p.resident ? tiles : 0);

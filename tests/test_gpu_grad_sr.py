@@ -432,3 +432,24 @@ def test_sr_products_wide_rows_and_many_rows(B, P):
     CU, a column group more or less) and, for many rows, on both sides of the
     rule for loads in flight."""
     test_sr_products_row_and_chunk_splits(B, P)
+
+
+@pytest.mark.parametrize('shape,per_cu', [((2, 2), 12), ((4, 4), 24)])
+def test_vjp_of_small_lattices_and_large_batches(rng, shape, per_cu):
+    """64 channels on one pixel tile: up to per_cu samples a CU in one kernel,
+    more in the other.  Against products with O in FP64; the bound of the tests
+    above."""
+    import flowket_amd as fk
+    cu = torch.cuda.get_device_properties(0).multi_processor_count
+    m = fk.ConvNetAutoregressive2D(shape, depth=3, num_of_channels=64, activation='elu', weights_normalization=False,
+                                   precision='fp32', seed=8)
+    B = per_cu * cu + 1
+    s = rng.choice([-1, 1], size=(B,) + shape).astype(np.int8)
+    u = torch.as_tensor(rng.normal(size=(B, 2)), device=m.device)
+    ref = torch.zeros(m.n_params, dtype=torch.float64, device=m.device)
+    for k in range(0, B, 512):
+        o_re, o_im, _ = m.per_sample_gradients(s[k:k + 512])
+        ref += u[k:k + 512, 0] @ o_re.double() + u[k:k + 512, 1] @ o_im.double()
+    for n, want in ((B, ref), (B - 1, ref - (u[-1, 0] * o_re[-1].double() + u[-1, 1] * o_im[-1].double()))):
+        got = m.vjp(s[:n], u[:n].float()).double()
+        assert (got - want).abs().max() < 2e-5 * want.abs().max()
