@@ -21,42 +21,71 @@ __device__ __forceinline__ WnLayer wn_layer(const int64_t* t, int l) {
 }
 
 // Threads of a workgroup over one (layer, tile of CT channels): channel
-// c = tile * CT + tid % CT, and the channel's nin values dealt to the G =
-// threads / CT groups tid / CT.  Neighbouring threads then read neighbouring
-// channels, so a wave's loads are contiguous (kernels are (..., cin, cout)).
-// What bounds these kernels is the chain of loads of one channel: with a
-// thread per channel it was nin (up to 576) dependent iterations, 213 us for
-// one row of the 4x4 depth-5 32-channel network and 519 us for 256 rows of
-// the 12x12 depth-10 one (1.6 TB/s); dealt to the groups, WN_FIGS.
+// c = tile * CT + tid % CT, and the channel's nin values dealt to G groups of
+// threads.  Neighbouring threads then read neighbouring channels, so a wave's
+// loads are contiguous (kernels are (..., cin, cout)).  What bounds these
+// kernels is the chain of loads of one channel: with a thread per channel it
+// was nin (up to 576) dependent iterations, 240 us for 64 rows of the 4x4
+// depth-5 32-channel network and 520 us for 256 rows of the 12x12 depth-10 one;
+// dealt to the groups, 32 and 283.
+// Networks of fewer than 16 channels have too few values for the threads, and
+// many rows would be as many nearly empty workgroups: there a group has four
+// values or more and the threads take several rows at a time (8192 rows, depth 3,
+// 2 channels: 24 us with a thread per channel, 593 with a row a workgroup, 26
+// so; depth 5, 8 channels 407, 658 and 349; 12 channels 831, 878 and 834; at
+// 16 channels one row a workgroup is the faster one, depth 6, 4096 rows: 733).
 constexpr int WN_THREADS = 256;
 
 struct WnTile {
-  int CT, G, grp;
+  int CT, G, rows;  // channels; groups; rows at a time
+  int col, grp, row;
   int64_t c;
   bool live;
 };
 
 __device__ __forceinline__ int wn_tile_channels(const WnLayer& L) { return L.cout < 64 ? (int)L.cout : 64; }
 
+// Groups of a row (1 .. WN_THREADS / CT): of four values or more, and as many
+// rows as come nearest to using all threads.
+__host__ __device__ inline int wn_row_groups(int CT, int64_t nin) {
+  const int all = WN_THREADS / CT;
+  const int most = nin < 8 ? 1 : nin / 4 < all ? (int)(nin / 4) : all;
+  const int rows = (2 * WN_THREADS / (CT * most) + 1) / 2;
+  const int even = WN_THREADS / (CT * rows);  // 0 where rounding up left no thread for a row
+  return even < 1 ? 1 : even < most ? even : most;
+}
+
+template <bool MULTI>
 __device__ __forceinline__ WnTile wn_tile(const WnLayer& L, int64_t tile) {
   WnTile t;
   t.CT = wn_tile_channels(L);
   t.G = WN_THREADS / t.CT;
+  t.rows = 1;
   t.grp = (int)threadIdx.x / t.CT;
-  t.c = tile * t.CT + (int)threadIdx.x % t.CT;
-  t.live = t.grp < t.G && t.c < L.cout;
+  t.row = 0;
+  t.col = (int)threadIdx.x % t.CT;
+  t.c = tile * t.CT + t.col;
+  if constexpr (MULTI) {
+    t.G = wn_row_groups(t.CT, L.nin);
+    t.rows = WN_THREADS / (t.CT * t.G);
+    t.row = t.grp / t.G;
+    t.grp -= t.row * t.G;
+    t.live = t.row < t.rows && t.c < L.cout;
+  } else {
+    t.live = t.grp < t.G && t.c < L.cout;
+  }
   return t;
 }
 
-// Sum over the groups of a channel, in group order (FP64, deterministic);
-// every thread of the channel gets it.  red: WN_THREADS doubles.
+// Sum over the groups of a channel (and row), in group order (FP64,
+// deterministic); every thread of the channel gets it.  red: WN_THREADS doubles.
 __device__ __forceinline__ double wn_group_sum(double x, const WnTile& t, double* red) {
   __syncthreads();
   red[threadIdx.x] = x;
   __syncthreads();
-  const int col = (int)threadIdx.x % t.CT;
+  const int first = (t.row < t.rows ? t.row : 0) * t.G * t.CT + t.col;
   double s = 0.0;
-  for (int k = 0; k < t.G; ++k) s += red[k * t.CT + col];
+  for (int k = 0; k < t.G; ++k) s += red[first + k * t.CT];
   return s;
 }
 
@@ -101,7 +130,7 @@ __global__ __launch_bounds__(WN_THREADS) void wn_effective_kernel(const float* _
   __shared__ double red[WN_THREADS];
   const WnLayer L = wn_layer(layers, blockIdx.y);
   if ((int64_t)blockIdx.x * wn_tile_channels(L) >= L.cout) return;
-  const WnTile t = wn_tile(L, blockIdx.x);
+  const WnTile t = wn_tile<false>(L, blockIdx.x);
   float n, s;
   bool clamped;
   wn_norm(v, L, t, g, exp_norm, red, n, s, clamped);
@@ -117,8 +146,9 @@ __global__ __launch_bounds__(WN_THREADS) void wn_effective_kernel(const float* _
 // kernel entries of every wrapped layer hold d/dv and row[P + goff + c] holds
 // d/dg.  dv_i = s/n (dk_i - v_i (v.dk)/n^2) (s/n dk_i when the norm is
 // clamped), dg = s/n (v.dk) for exponential_norm, (v.dk)/n otherwise.  A
-// workgroup takes rows blockIdx.z, blockIdx.z + gridDim.z, ... of one (tile,
-// layer), so the norm is computed once for them.
+// workgroup takes sets of t.rows rows, blockIdx.z, blockIdx.z + gridDim.z, ...,
+// of one (tile, layer), so the norm is computed once for them.
+template <bool MULTI>
 __global__ __launch_bounds__(WN_THREADS) void wn_grad_rows_kernel(float* __restrict__ rows, int64_t nrows, int64_t ld,
                                                                   const float* __restrict__ v,
                                                                   const float* __restrict__ g,
@@ -127,15 +157,20 @@ __global__ __launch_bounds__(WN_THREADS) void wn_grad_rows_kernel(float* __restr
   __shared__ double red[WN_THREADS];
   const WnLayer L = wn_layer(layers, blockIdx.y);
   if ((int64_t)blockIdx.x * wn_tile_channels(L) >= L.cout) return;
-  const WnTile t = wn_tile(L, blockIdx.x);
+  const WnTile t = wn_tile<MULTI>(L, blockIdx.x);
   float n, s;
   bool clamped;
   wn_norm(v, L, t, g, exp_norm, red, n, s, clamped);
   const float sn = s / n;
-  for (int64_t r = blockIdx.z; r < nrows; r += gridDim.z) {
-    float* row = rows + r * ld;
+  for (int64_t r0 = (int64_t)blockIdx.z * t.rows; r0 < nrows; r0 += (int64_t)gridDim.z * t.rows) {
+    bool live = t.live;
+    float* row = rows + r0 * ld;
+    if constexpr (MULTI) {
+      live = live && r0 + t.row < nrows;
+      if (live) row += t.row * ld;
+    }
     const float dot = wn_dot(v, row, L, t, red);
-    if (!t.live) continue;
+    if (!live) continue;
     const float proj = clamped ? 0.0f : dot / (n * n);
 #pragma unroll 4
     for (int64_t i = t.grp; i < L.nin; i += t.G) {
@@ -162,7 +197,7 @@ __global__ __launch_bounds__(WN_THREADS) void wn_tangent_kernel(const float* __r
   __shared__ double red[WN_THREADS];
   const WnLayer L = wn_layer(layers, blockIdx.y);
   if ((int64_t)blockIdx.x * wn_tile_channels(L) >= L.cout) return;
-  const WnTile t = wn_tile(L, blockIdx.x);
+  const WnTile t = wn_tile<false>(L, blockIdx.x);
   float n, s;
   bool clamped;
   wn_norm(v, L, t, g, exp_norm, red, n, s, clamped);
@@ -196,7 +231,7 @@ int fk_wn_grad_rows(float* rows, int64_t nrows, int64_t ld, const float* params,
   // few rows: a workgroup per row; many: the rows dealt to as many workgroups
   // as keep 16 of them per CU, so that the norms are not recomputed per row
   const int64_t most = 1 + 16LL * device_cu_count() / n_layers;
-  hipLaunchKernelGGL(wn_grad_rows_kernel,
+  hipLaunchKernelGGL((max_cout < 16 ? wn_grad_rows_kernel<true> : wn_grad_rows_kernel<false>),
                      dim3((unsigned)div_up(max_cout, 64), (unsigned)n_layers, (unsigned)(nrows < most ? nrows : most)),
                      dim3(WN_THREADS), 0, (hipStream_t)stream, rows, nrows, ld, params, g, layers, exp_norm, n_params);
   FK_CHECK_LAUNCH();

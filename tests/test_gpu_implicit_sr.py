@@ -362,3 +362,43 @@ def test_effective_params_first_called_under_capture():
         g.replay()
         torch.cuda.synchronize()
         assert torch.equal(out, eager.effective_params())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('exp_norm', [True, False])
+@pytest.mark.parametrize('channels,nrows', [(2, 1), (2, 77), (2, 6000), (6, 1000), (10, 333), (16, 65), (32, 300),
+                                            (64, 7), (100, 5)])
+def test_wn_gradient_rows(rng, channels, nrows, exp_norm):
+    """fk_wn_grad_rows on rows of random d/dk against the chain rule in FP64,
+    where a workgroup takes one row or several and the last set is not full.
+    Tolerance: v.dk is rounded once (2^-24 of its size, at most |v| |dk|), then a
+    few FP32 operations: 1e-6 of |s/n| (|dk| + |v| |v.dk| / n^2) per entry."""
+    import flowket_amd as fk
+    m = fk.ConvNetAutoregressive2D((3, 3), depth=3, num_of_channels=channels, weights_normalization=True,
+                                   exponential_norm=exp_norm, seed=7)
+    m.set_wn_g(m.wn_g + 0.3 * torch.randn(m.wn_g.shape, device=m.device))
+    P, G = m.n_params, m.wn_g.numel()
+    rows = torch.randn((nrows, P + G + 3), device=m.device)
+    got = rows.clone()
+    m._wn_rows(got, nrows)
+    assert torch.equal(got[:, P + G:], rows[:, P + G:])
+    p, g, off, goff = m.params.double(), m.wn_g.double(), 0, 0
+    for k, (ks, bs) in enumerate(m.shapes):
+        nk, c = int(np.prod(ks)), bs[0]
+        dk = rows[:, off:off + nk].double().reshape(nrows, -1, c)
+        if k == len(m.shapes) - 1:
+            assert torch.equal(got[:, off:off + nk + c], rows[:, off:off + nk + c])
+            break
+        v = p[off:off + nk].reshape(-1, c)
+        n = v.norm(dim=0)
+        s = torch.exp(g[goff:goff + c]) if exp_norm else g[goff:goff + c]
+        dot, size = (v * dk).sum(dim=1), (v.abs() * dk.abs()).sum(dim=1)
+        want = s / n * (dk - v * (dot / n ** 2)[:, None])
+        scale = (s / n).abs() * (dk.abs() + v.abs() * (size / n ** 2)[:, None])
+        err = (got[:, off:off + nk].double().reshape(nrows, -1, c) - want).abs()
+        assert (err <= 1e-6 * scale).all()
+        err = (got[:, P + goff:P + goff + c].double() - (s / n * dot if exp_norm else dot / n)).abs()
+        assert (err <= 1e-6 * (s / n if exp_norm else 1 / n).abs() * size).all()
+        assert torch.equal(got[:, off + nk:off + nk + c], rows[:, off + nk:off + nk + c])
+        off += nk + c
+        goff += c
