@@ -9,6 +9,8 @@ normalisation (deepar/layers/wrappers.py:123-135) is a per-step transform of
 that vector.  Every evaluation runs in the fused forward kernel
 (fk_convar_forward).
 """
+import math
+
 import numpy as np
 import torch
 
@@ -525,11 +527,11 @@ class ConvNetAutoregressive2D:
         if getattr(self, '_wn_tab', None) is None:
             rows, off, goff = [], 0, 0
             for idx, (kshape, bshape) in enumerate(self.shapes):
-                nk = int(np.prod(kshape))
+                nk = math.prod(kshape)
                 if idx < len(self.shapes) - 1:
                     rows.append([off, nk // kshape[3], kshape[3], goff])
                     goff += kshape[3]
-                off += nk + int(np.prod(bshape))
+                off += nk + bshape[0]
             tab = torch.as_tensor(np.asarray(rows, dtype=np.int64)).to(self.device)
             self._wn_tab = (tab, len(rows), max(r[2] for r in rows))
         return self._wn_tab
