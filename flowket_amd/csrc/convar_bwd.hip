@@ -13,8 +13,9 @@
 // (relu' = [y > 0], elu' = y > 0 ? 1 : y + 1).
 //
 // 32 and 64 channels take convar_grad.hip (grad_plan); this file's MFMA kernels
-// the larger multiples of 32, and operands that are not aligned to 16 bytes;
-// the scalar kernel the other widths.
+// the larger multiples of 32, operands that are not aligned to 16 bytes, lattices
+// whose tables do not fit that kernel's LDS, and the VJP of small lattices of 64
+// channels in large batches; the scalar kernel the other widths.
 #include "convar_bwd.h"
 
 #include <algorithm>

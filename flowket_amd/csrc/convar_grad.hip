@@ -1,7 +1,7 @@
 // Gradients of log psi of ConvNetAutoregressive2D (32 and 64 channels): the
 // per-sample rows O_k, their batched adjoint product (VJP) and forward mode
 // (JVP), FP32 MFMA.  Same quantities as convar_bwd.hip, which keeps the other
-// channel counts.
+// channel counts and what grad_plan leaves it.
 //
 // One workgroup per sample at a time, its waves sharing every phase.  A block
 // of the network is two phases, forward and backward, with one barrier each:
@@ -14,10 +14,11 @@
 //            VH: the weight gradients of the 1x1s and of the V and H
 //                convolutions, and their data gradients
 // The activations' derivatives, biases and residuals run in the epilogues.
-// Five tensors of the sample (HW x C, FP32) are live in either direction; when
-// they fit they stay in LDS (RES), with rows of C + 4 floats (the 16 pixels of
-// a tile then start 36 or 68 banks apart) and a zero pixel that taps outside
-// the lattice read.  The activations that the backward needs go to the
+// Five tensors of the sample (HW x C, FP32) are live in either direction, eight
+// in the JVP; when they fit they stay in LDS (RES: up to 192 pixels at C 32, 108
+// at C 64; JVP 127 and 67), with rows of C + 4 floats (the 16 pixels of a tile
+// then start 36 or 68 banks apart) and a zero pixel that taps outside the lattice
+// read.  The activations that the backward needs go to the
 // workgroup's workspace.  Larger lattices keep all tensors there (L2).
 //
 // The bound is the matrix cores (FP32 MFMA, 32 cycles each), of which a phase
@@ -27,11 +28,11 @@
 // weights, and requests between the MFMAs of the step before.  With a phase
 // per convolution and one elementwise pass per derivative (13 barriers a
 // block, four waves) the matrix cores were busy a quarter of the time.
-// Measured, VJP / JVP / O in ms, before -> now: 10x10 depth 20 C 32, 64
-// samples 5.86 / 3.81 / 9.21 -> 1.91 / 1.45 / 3.08; 2048 samples 25.4 / 19.7 /
-// samples 5.86 / 3.81 / 9.21 / 11.5 / 24.8; 20x20 depth 24 C 64,
-// 128 samples 88.6 / 56.3 / 155.9 -> 27.6 / 22.5 / 45.2; 4x4 depth 5 C 32, 1024
-// samples 1.54 / 0.66 / 1.23 -> 0.65 / 0.21 / 0.74.
+// Measured, VJP / JVP / O in ms, convar_bwd.hip -> here: 10x10 depth 20 C 32, 64
+// samples 5.86 / 3.81 / 9.21 -> 1.87 / 1.43 / 3.06, 2048 samples 25.2 / 19.6 /
+// 36.1 -> 15.7 / 11.4 / 24.8; 20x20 depth 24 C 64, 128 samples 88.6 / 56.3 /
+// 155.9 -> 27.6 / 22.5 / 45.2, 512 samples 141 / 100 / 238 -> 56.6 / 45.5 / 92.2;
+// 4x4 depth 5 C 32, 1024 samples 1.55 / 0.64 / 1.23 -> 0.72 / 0.20 / 0.72.
 #include "convar_bwd.h"
 
 namespace fk {
@@ -1124,11 +1125,11 @@ GradPlan grad_plan(const BwdArgs& a, int mode) {
   // small lattices, with fewer units in a phase than waves, run two or four to
   // a CU once the batch has a sample for each.  Not the VJP: every workgroup
   // adds a row of partial sums for the reduction.  1024 samples, ms: 4x4 C 32
-  // O 0.94 at one, 0.74 at four, JVP 0.48 and 0.22, but VJP 0.70 and 1.15; 8x8
-  // C 32 O 2.20 at one, 2.06 at two.  1024 threads (one pixel tile a unit)
-  // against 512 (two): 10x10 C 32, 2048 samples, VJP 15.6 and 16.6, O 24.7 and
-  // 26.6, JVP 11.4 both; C 64 has no registers for 1024 (10x10, 1024 samples,
-  // VJP 14.4 and 13.0).
+  // O 0.94 at one, 0.74 at four, JVP 0.48 and 0.22, but VJP (a row a workgroup)
+  // 0.70 and 1.15; 8x8 C 32 O 2.20 at one, 2.06 at two.  1024 threads (one pixel
+  // tile a unit) against 512 (two): 10x10 C 32, 2048 samples, VJP 15.6 and 16.6, O
+  // 24.7 and 26.6, JVP 11.4 both; C 64 has no registers for 1024 (10x10, 1024
+  // samples, VJP 14.4 and 13.0).
   p.threads = p.resident ? resident_threads(C, mode) : 512;
   p.per_cu = 1;
   if (p.resident && mode != GRAD_VJP) {

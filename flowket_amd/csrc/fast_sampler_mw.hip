@@ -29,12 +29,12 @@
 // operations at the start of each super-tick, so a store issued in J is
 // complete when barrier J + 1 has passed, and requests made at the end of K
 // see the outputs that the chain made in K - 3 or before.  An operand of a
-// step is at least nb steps older than it, so nb >= 5 G suffices (G is at
-// most that); between 4 G and 5 G the helpers also wait for their stores
-// before the barrier, which saves one super-tick.  Networks of two blocks,
-// FP32 networks of 64 channels (their fragments are single floats: spills,
-// 226 against 144 ms for 64 10x10 samples) and rows wider than the LDS take
-// the one-wave kernel.
+// step is at least nb steps older than it, so nb >= 5 G suffices; between 4 G
+// and 5 G (G is at most nb / 4) the helpers also wait for their stores before
+// the barrier, which saves one super-tick.  Networks of two blocks, FP32
+// networks of 64 channels (their fragments are single floats: spills, 226
+// against 144 ms for 64 10x10 samples), rows wider than the LDS and the calls
+// that fast_mw_takes leaves take the one-wave kernel.
 //
 // Measured (one wave per 16 samples -> this kernel):
 //   20x20 depth 24 C64 bf16, 512 samples    204.3 -> 26.6 ms
@@ -42,9 +42,10 @@
 //   10x10 depth 20 C32 fp16, 64 / 1024 / 8192  4.7 -> 2.2, 4.8 -> 2.5, 7.4 -> 6.7 ms
 //   10x10 depth 20 C32 fp32, 1024 / 8192      43 -> 9.1, 54 -> 19 ms
 //   10x10 depth 5 C32 fp16, 64 / 8192       0.96 -> 0.56, 1.67 -> 1.50 ms
-// A chain step takes about 790 cycles at 16-bit C32 and 1960 at C64 (one wave
-// issuing its instructions); at two tiles per CU (8192 samples) the cache's
-// traffic to HBM bounds the C32 kernel.
+// A chain step takes 334 ns (774 cycles) at 16-bit C32 and 793 ns (1907) at C64
+// (16 samples of a single row, 60 and 34 sites, depth 20), the issue of one
+// wave's instructions.  At two tiles per CU (8192 10x10 samples) the cache's
+// traffic beyond L2 bounds it: 36 GB in 6.9 ms, 5.3 TB/s, a copy's rate.
 #include "fast_sampler.h"
 
 #include <type_traits>
@@ -103,7 +104,7 @@ __global__ __launch_bounds__((64 * Mw<PREC, C>::NW), (Mw<PREC, C>::WPE)) void fa
   // cache of the tile, as in fast_sampler.hip: HW pixels per buffer (two more
   // unused).  Taps outside the lattice are loaded like the others, from
   // whatever lies there (so a row of taps is one scalar offset and constants),
-  // and replaced by zeros; MW_PAD pixels before the first buffer keep those
+  // and replaced by zeros; mw_pad pixels before the first buffer keep those
   // loads inside the cache.
   uint8_t* base = a.cache + (int64_t)blockIdx.x * a.tile_bytes;
   const int BUF = (HW + 2) * PB;
@@ -795,7 +796,7 @@ __global__ __launch_bounds__((64 * Mw<PREC, C>::NW), (Mw<PREC, C>::WPE)) void fa
   }
 }
 
-// Steps per super-tick: one per helper, a fifth of the blocks at most, and
+// Steps per super-tick: one per helper, a quarter of the blocks at most, and
 // what the LDS holds.
 constexpr int MW_LDS = 160 * 1024;
 

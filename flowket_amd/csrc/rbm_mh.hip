@@ -4,11 +4,11 @@
 // layers/complex/tensorflow_ops.py:69-85):
 //   log psi(s) = sum_j a_j s_j + sum_h lncosh(theta_h),  theta_h = b_h + sum_j W_jh s_j,
 // complex parameters stored as (real, imag) pairs and used as real - 1j*imag
-// (layers/complex/base_layer.py:30-35).  One wavefront per configuration, the
-// hidden units spread over the lanes.
+// (layers/complex/base_layer.py:30-35).  A wavefront evaluates one configuration
+// or eight, the hidden units spread over the lanes.
 //
-// MH (samplers/metropolis_hastings.py:15-145): one wavefront per chain keeps
-// theta in registers and updates it incrementally for each accepted move
+// MH (samplers/metropolis_hastings.py:15-145): a workgroup of one to eight waves
+// per chain keeps theta in registers and updates it for each accepted move
 // (a flipped site s_j changes theta by -2 s_j W_j.), so a proposal costs
 // O(M) instead of a full O(N M) evaluation.  Acceptance is the reference rule
 // exp(min(2 Re(logpsi' - logpsi), 0)) > U.  Random numbers are either

@@ -9,7 +9,8 @@
 
 namespace fk {
 
-// Column kernels (o_mean, oh_times_u): a wave owns 64 x 4 consecutive columns
+// Column kernels (o_mean, and oh_times_u where the columns alone do not fill the
+// chip): a wave owns 64 x 4 consecutive columns
 // (one 16-byte load per lane, row and part) and the rows are dealt to the
 // waves of a workgroup in contiguous ranges, whose FP64 sums are added in
 // wave order through LDS.  HBM bound: with one thread per column group over
@@ -390,7 +391,7 @@ __global__ void oh_times_u_kernel(const float* __restrict__ ore, const float* __
 // Job B re-reads rows that job A of the previous launch streamed in, so with
 // two blocks in flight (2 R rows x 2 parts x 4 P bytes) inside the 256 MB
 // last-level cache the second read does not reach HBM.  (Measured at B = 8192,
-// P = 849,156: 20.0 ms at R = 16 against 18.9 ms for the two HBM passes --
+// P = 849,156: 20.0 ms at R = 16 against 18.7 ms for the two HBM passes --
 // reads served by the last-level cache come no faster than HBM streams, so
 // the two-pass form stays the default.)  The kernel boundary
 // between the launches orders job A's partials before job B's reads; every
@@ -738,7 +739,8 @@ int fk_oh_times_u(const float* o_re, const float* o_im, const float* mean_re, co
     const int64_t p4 = n_params / 4;
     const OhArgs a{reinterpret_cast<const f32x4*>(o_re), reinterpret_cast<const f32x4*>(o_im), mean_re, mean_im, u,
                    scratch2, batch, p4, scale, shift, v, out};
-    // By waves of columns per CU: from 10 on they need no second range of rows,
+    // By waves of columns per CU: from 10 on they need no second range of rows
+    // (from 12 on two waves a workgroup, 849,156 columns; below one is faster),
     // from 7 on two ranges do, with registers for eight waves per SIMD; fewer are
     // dealt as in o_mean.  (A thread per four columns over all rows / dealt as in
     // o_mean / this, ms: 8192 rows x 849,156 9.59 / 10.03 / 9.47, x 700,000 7.63 /

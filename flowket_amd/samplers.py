@@ -90,8 +90,9 @@ class AutoregressiveSampler(Sampler):
 class FastAutoregressiveSampler(AutoregressiveSampler):
     """deepar/samplers/fast_autoregressive.py:13-76: same distribution and,
     given the same uniforms, the same draws as AutoregressiveSampler, with each
-    (layer, site) activation computed once (fk_fast_sample: one wavefront per
-    16 samples walking the lattice, activation cache in device memory).
+    (layer, site) activation computed once (fk_fast_sample: a workgroup of four
+    waves or one wave per 16 samples walking the lattice, activation cache in
+    device memory).
     ``mini_batch_size`` bounds the cache: batches larger than it are drawn in
     chunks (:30-35)."""
 
